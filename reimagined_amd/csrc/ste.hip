@@ -1,0 +1,595 @@
+// The packed BitLinear straight-through backward (src/bitlinear.cpp:1191-1357 of
+// vitorGgC569/reimagined, OXN/nsos/): dW, dx, the magnitude and bias gradients.
+//
+// Both contractions have one f32 operand (the gradient) and one operand that bf16
+// holds exactly: the int8 codes (|q| <= 127, 7 bits) and the ternary weights.  The
+// f32 operand is cut into three bf16 pieces (8 + 8 + 8 significant bits: their sum
+// is the value), so three v_mfma_f32_32x32x16_bf16 with f32 accumulation give the
+// products that v_mfma_f32_32x32x2_f32 gives, each exact before it is added, at a
+// sixteenth of the matrix-core time per pass.  Before: two fp32-MFMA GEMMs at the
+// card's fp32 rate (400 + 407 us at M = 4096, K = 1024, N = 4096), a full ternary
+// GEMM for dmag (27 us) and a column reduction over two [M, N] arrays (145 us).  Now one
+// launch of 213 us for both contractions and the column sums (MFMA issue alone: 94 us at
+// the ~2.1 GHz it runs at; dW's strided gradient reads and its epilogue make its tiles the
+// longer ones), a forward and backward step 1061 -> 267 us.
+#include "common.hpp"
+
+#include <cmath>
+
+namespace nsosx {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+constexpr int kTR = 128, kTC = 256;           // output tile: gradient rows x exact columns
+constexpr int kTK = 32;                       // reduction depth of one LDS stage
+constexpr int kSteThreads = 512;              // eight waves of 64 x 64, 2 x 4
+constexpr int kPlane = kTR * kTK * 2;         // bytes of one gradient piece of a stage
+constexpr int kSteStage = 3 * kPlane + kTC * kTK * 2;
+constexpr int kSteSmem = 2 * kSteStage;       // double buffered: 80 KB
+
+struct SteArgs {
+    const float* grad;       // [M, N]
+    const float* mag;        // [N] or null
+    const float* as;         // [M]
+    const uint16_t* qT;      // bf16 [K][Mp]: the codes, reduction-contiguous, zero past M
+    const uint16_t* tT;      // bf16 [K][Np]: the ternary weights, zero past N
+    const uint32_t* packed;  // [N, K / 16]
+    const float* wlat;       // [N, K]
+    float* dW;               // [N, K]
+    float* dact;             // [M, K]
+    float* part_mag;         // [4 * K tiles][N] or null
+    float* dbias;            // [N] or null
+    float ws, clip;
+    int M, K, N, Mp, Np;
+};
+
+// 16-byte chunk c (8 reduction elements) of tile row r: swizzled so that the 16 rows
+// a fragment read serves per clock cover all 64 banks.
+__device__ __forceinline__ int tile_at(int r, int c) { return r * 64 + ((c ^ ((r >> 2) & 3)) << 4); }
+
+// Two floats -> three pairs of bf16 pieces, by truncation: hi holds the top
+// 8 significant bits, the remainders are exact.  GUARD: an infinity goes whole into hi
+// (its remainder would be NaN).  A NaN stays one in every piece (the hardware's NaNs
+// are quiet).
+template <bool GUARD>
+__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& hi, uint32_t& mid,
+                                            uint32_t& lo) {
+    float r0 = __fsub_rn(x0, __uint_as_float(__float_as_uint(x0) & 0xffff0000u));
+    float r1 = __fsub_rn(x1, __uint_as_float(__float_as_uint(x1) & 0xffff0000u));
+    if (GUARD && fabsf(x0) == __builtin_inff()) r0 = 0.0f;
+    if (GUARD && fabsf(x1) == __builtin_inff()) r1 = 0.0f;
+    const float l0 = __fsub_rn(r0, __uint_as_float(__float_as_uint(r0) & 0xffff0000u));
+    const float l1 = __fsub_rn(r1, __uint_as_float(__float_as_uint(r1) & 0xffff0000u));
+    hi = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
+    mid = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    lo = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), 0x07060302u);
+}
+
+// One 128 x 256 output tile: acc[rows][cols] = sum over the reduction of the gradient
+// operand (rows o0 .. of dW's j or d_act's m) and the exact operand bT (columns k0 ..).
+// DW: the gradient is read [reduction][output] (grad columns j, scaled by as[i]); else
+// [output][reduction] (grad rows m, scaled by mag[j]).  A thread cuts 8 reduction
+// elements of one tile row per stage.  The whole stages run branch-free (rows and columns
+// past the operands re-read the last: their outputs are never stored), the split's VALU
+// between the MFMAs and the loads two stages ahead; a last stage cut by the reduction's
+// end, and a tile that meets an infinity, go through slow_stage().
+// colsum (DW): the thread's share of sum_i grad[i][j] for its column.
+template <bool DW, bool MAG>
+__device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char* smem,
+                                         v16f (&acc)[2][2], float& colsum) {
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int red = DW ? g.M : g.N;
+    const int full = red / kTK;
+    const uint16_t* bT = DW ? g.qT : g.tT;
+    const int ldb = DW ? g.Mp : g.Np;
+    // exact operand: columns tid / 4 and + 128, chunk tid % 4
+    const uint16_t* bsrc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        bsrc[i] = bT + (int64_t)min(k0 + (tid >> 2) + 128 * i, g.K - 1) * ldb + (tid & 3) * 8;
+    // gradient: DW column tid % 128, reduction chunk tid / 128 (the same for a whole wave);
+    // else row tid / 4, chunk tid % 4
+    const int row = DW ? tid & 127 : tid >> 2;
+    const int chunk = DW ? wave >> 1 : tid & 3;
+    const int orow = min(o0 + row, (DW ? g.N : g.M) - 1);
+    const float* asrc = DW ? g.grad + orow : g.grad + (int64_t)orow * g.N;
+
+    struct Stage {
+        float f[8], sc[8];
+        u32x4 b[2];
+    };
+    auto load = [&](int st, Stage& s) {
+        const int r0 = min(st, full - 1) * kTK;  // (past the end: the last again, not used)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) s.b[i] = *reinterpret_cast<const u32x4*>(bsrc[i] + r0);
+        const int n = r0 + chunk * 8;
+        if constexpr (DW) {
+            const float* p = asrc + (int64_t)n * g.N;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s.f[e] = p[(int64_t)e * g.N];
+            __builtin_memcpy(s.sc, g.as + n, 32);  // (4-byte aligned)
+        } else {
+            __builtin_memcpy(s.f, asrc + n, 32);
+            if (MAG) __builtin_memcpy(s.sc, g.mag + n, 32);
+        }
+    };
+    const int a_at = tile_at(row, chunk);
+    float top = 0.0f;
+    auto put = [&](char* dst, const u32x4 (&piece)[3]) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPlane + a_at) = piece[p];
+    };
+    auto put_b = [&](char* dst, const Stage& s) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            *reinterpret_cast<u32x4*>(dst + 3 * kPlane + tile_at((tid >> 2) + 128 * i, tid & 3)) = s.b[i];
+    };
+    auto cut = [&](const Stage& s, int p, u32x4 (&piece)[3]) {  // elements 2p, 2p + 1
+        const float v0 = DW || MAG ? __fmul_rn(s.f[2 * p], s.sc[2 * p]) : s.f[2 * p];
+        const float v1 = DW || MAG ? __fmul_rn(s.f[2 * p + 1], s.sc[2 * p + 1]) : s.f[2 * p + 1];
+        top = fmaxf(top, fmaxf(fabsf(v0), fabsf(v1)));
+        uint32_t h, m, l;
+        split3_pair<false>(v0, v1, h, m, l);
+        piece[0][p] = h; piece[1][p] = m; piece[2][p] = l;
+    };
+    auto add_cols = [&](const Stage& s, bool on) {
+        const float t = ((s.f[0] + s.f[1]) + (s.f[2] + s.f[3])) + ((s.f[4] + s.f[5]) + (s.f[6] + s.f[7]));
+        colsum += on ? t : 0.0f;
+    };
+    const int wm = wave >> 2, wn = wave & 3;
+    const int li = lane & 31, lh = lane >> 5;
+    // A stage is six steps of four MFMAs: two 16-deep k steps x three pieces, the smallest
+    // first; fragment a(step) of the pieces, b(k step) of the exact operand.
+    auto frag_b = [&](const char* s, int ks, v8bf (&b)[2]) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+            b[n] = *reinterpret_cast<const v8bf*>(s + 3 * kPlane +
+                                                  tile_at(wn * 64 + n * 32 + li, 2 * ks + lh));
+    };
+    auto frag_a = [&](const char* s, int step, v8bf (&a)[2]) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            a[m] = *reinterpret_cast<const v8bf*>(
+                s + (2 - step % 3) * kPlane + tile_at(wm * 64 + m * 32 + li, 2 * (step / 3) + lh));
+    };
+    auto mfma4 = [&](const v8bf (&a)[2], const v8bf (&b)[2]) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+                acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[m], b[n], acc[m][n], 0, 0, 0);
+    };
+    // a step's fragment reads, then its MFMAs with VALU work in their shadow (left alone the
+    // compiler clusters the MFMAs behind single reads and the cuts before them)
+    auto fence = [&]() {
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Stage st from LDS, its first fragments already in a[0], b[0]; meanwhile stage st + 1 (in
+    // s) is cut and written, and s reloaded.  The barrier stands before the last step's
+    // MFMAs, whose fragments are in registers: they cover the next stage's first reads.
+    v8bf a[2][2], b[2][2];
+    auto advance = [&](int st, Stage& s) {
+        const char* cur = smem + (st & 1) * kSteStage;
+        char* nxt = smem + ((st + 1) & 1) * kSteStage;
+        u32x4 piece[3];
+#pragma unroll
+        for (int step = 0; step < 5; ++step) {
+            if (step == 1) frag_b(cur, 1, b[1]);
+            frag_a(cur, step + 1, a[(step + 1) & 1]);
+            mfma4(a[step & 1], b[step / 3]);
+            if (step < 4) cut(s, step, piece);
+            if (step == 4) {
+                put(nxt, piece);
+                put_b(nxt, s);
+            }
+            fence();
+        }
+        __syncthreads();
+        frag_b(nxt, 0, b[0]);
+        frag_a(nxt, 0, a[0]);
+        mfma4(a[1], b[1]);
+        if (DW) add_cols(s, st + 1 < full);
+        load(st + 3, s);
+        fence();
+    };
+    auto slow_stage = [&](int st, bool cols) {
+        Stage s;
+        const int n = st * kTK + chunk * 8;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int at = min(n + e, red - 1);
+            const float f = asrc[DW ? (int64_t)at * g.N : (int64_t)at];
+            const float sc = DW ? g.as[at] : (MAG ? g.mag[at] : 1.0f);
+            s.f[e] = n + e < red ? f : 0.0f;
+            v[e] = n + e < red ? __fmul_rn(f, sc) : 0.0f;
+            top = fmaxf(top, fabsf(v[e]));
+        }
+        if (DW) add_cols(s, cols);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) s.b[i] = *reinterpret_cast<const u32x4*>(bsrc[i] + st * kTK);
+        u32x4 piece[3];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            uint32_t h, m, l;
+            split3_pair<true>(v[2 * p], v[2 * p + 1], h, m, l);
+            piece[0][p] = h; piece[1][p] = m; piece[2][p] = l;
+        }
+        put(smem, piece);
+        put_b(smem, s);
+        __syncthreads();
+#pragma unroll
+        for (int step = 0; step < 6; ++step) {
+            if (step % 3 == 0) frag_b(smem, step / 3, b[0]);
+            frag_a(smem, step, a[0]);
+            mfma4(a[0], b[0]);
+        }
+        __syncthreads();
+    };
+
+    if (full > 0) {
+        Stage s0, s1;
+        // (the fences keep each set's loads together, so that waiting for one set leaves the
+        // other's in flight)
+        load(0, s0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(1, s1);
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 piece[3];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) cut(s0, p, piece);
+        put(smem, piece);
+        put_b(smem, s0);
+        if (DW) add_cols(s0, true);
+        __builtin_amdgcn_sched_barrier(0);
+        load(2, s0);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        frag_b(smem, 0, b[0]);
+        frag_a(smem, 0, a[0]);
+        // stage st is in LDS, st + 1 and st + 2 in s1 / s0 (in flight); a stage past the end
+        // is written to the buffer that nothing reads any more
+        int st = 0;
+        for (; st + 1 < full; st += 2) {
+            advance(st, s1);
+            advance(st + 1, s0);
+        }
+        if (st < full) advance(st, s1);
+        __syncthreads();  // (the stage past the end was read, though not used)
+    }
+    if (full * kTK < red) slow_stage(full, true);
+    if (__syncthreads_or(top == __builtin_inff())) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[i][n] = v16f{};
+        for (int st = 0; st * kTK < red; ++st) slow_stage(st, false);
+    }
+}
+
+// dW and d_act tiles in one launch (each alone is 128 tiles at 4096 x 1024, together one
+// for each CU).  An XCD gets a run of consecutive tiles, K tiles fastest, so that the
+// tiles sharing a gradient panel share an L2.
+__global__ __launch_bounds__(kSteThreads, 2) void ste_gemm_kernel(SteArgs g) {
+    extern __shared__ __align__(16) char smem_ste[];
+    const int tk = (g.K + kTC - 1) / kTC;
+    const int tiles_w = ((g.N + kTR - 1) / kTR) * tk;
+    const int total = gridDim.x;
+    const int per = total / 8;
+    int t = blockIdx.x;
+    if (t < per * 8) t = (t % 8) * per + t / 8;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 2, wn = wave & 3;
+    const int li = lane & 31, lh = lane >> 5;
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) acc[i][n] = v16f{};
+    float colsum = 0.0f;
+    const int k0 = (t < tiles_w ? t % tk : (t - tiles_w) % tk) * kTC;
+
+    // D layout of the 32x32 MFMA: register r of lane l holds row 8 (r / 4) + 4 (l / 32) +
+    // r % 4, column l % 32
+    if (t >= tiles_w) {
+        const int m0 = (t - tiles_w) / tk * kTR;
+        if (g.mag) ste_tile<false, true>(g, m0, k0, smem_ste, acc, colsum);
+        else ste_tile<false, false>(g, m0, k0, smem_ste, acc, colsum);
+        const bool whole = m0 + kTR <= g.M && k0 + kTC <= g.K;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                const int k = k0 + wn * 64 + n * 32 + li;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+                    if (whole || (m < g.M && k < g.K))
+                        g.dact[(int64_t)m * g.K + k] = __fmul_rn(acc[i][n][r], g.ws);
+                }
+            }
+        return;
+    }
+
+    const int j0 = t / tk * kTR;
+    // dbias of the tile's columns: the four chunks' shares (the K tiles all read the same
+    // gradient columns; the first one sums and stores)
+    const bool sums = g.dbias && k0 == 0;
+    ste_tile<true, false>(g, j0, k0, smem_ste, acc, colsum);
+    if (sums) {
+        float* s = reinterpret_cast<float*>(smem_ste);  // idle: the last stage ended in a barrier
+        s[tid] = colsum;
+        __syncthreads();
+        if (tid < kTR && j0 + tid < g.N)
+            g.dbias[j0 + tid] = ((s[tid] + s[kTR + tid]) + s[2 * kTR + tid]) + s[3 * kTR + tid];
+    }
+    // per 32 rows: the latent weights, the packed words and the magnitudes of the wave's
+    // outputs loaded together, clamped into the matrix (each under its own branch they came
+    // one at a time: 90 us of 232).  |w / clip| > 1 after rounding is |w| > clip: the next
+    // float above clip already divides to more than 1 + 2^-24.
+    const bool whole = j0 + kTR <= g.N && k0 + kTC <= g.K;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int jr = j0 + wm * 64 + i * 32 + 4 * lh;  // row r at + 8 (r / 4) + r % 4
+        float wl[2][16], mg[16];
+        uint32_t words[2][16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int j = min(jr + 8 * (r >> 2) + (r & 3), g.N - 1);
+            mg[r] = g.mag ? g.mag[j] : 1.0f;
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                const int64_t at = (int64_t)j * g.K + min(k0 + wn * 64 + n * 32 + li, g.K - 1);
+                wl[n][r] = g.wlat[at];
+                words[n][r] = g.part_mag ? g.packed[at >> 4] : 0u;  // K % 16 == 0
+            }
+        }
+        float dm[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int j = jr + 8 * (r >> 2) + (r & 3);
+            dm[r] = 0.0f;
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                const int k = k0 + wn * 64 + n * 32 + li;
+                const float v = acc[i][n][r];
+                const uint32_t c = (words[n][r] >> (2 * (k & 15))) & 3u;
+                if (k < g.K) dm[r] += c == 0u ? -v : (c == 2u ? v : 0.0f);
+                const float d = fabsf(wl[n][r]) > g.clip ? 0.0f : __fmul_rn(v, mg[r]);
+                if (whole || (j < g.N && k < g.K)) g.dW[(int64_t)j * g.K + k] = d;
+            }
+        }
+        if (g.part_mag) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {  // over the 32 columns
+                dm[r] += lane_xor<16>(dm[r]);
+                dm[r] += lane_xor<8>(dm[r]);
+                dm[r] += lane_xor<4>(dm[r]);
+                dm[r] += lane_xor<2>(dm[r]);
+                dm[r] += lane_xor<1>(dm[r]);
+                const int j = jr + 8 * (r >> 2) + (r & 3);
+                if (j < g.N && li == 0) g.part_mag[(int64_t)(4 * (k0 / kTC) + wn) * g.N + j] = dm[r];
+            }
+        }
+    }
+}
+
+// dmag[j] = sum_i grad[i][j] * pre[i][j] with pre = acc * (as * ws), taken as
+// ws * sum_k T[j][k] G[j][k] from the dW tiles' G = sum_i grad * as * q.  Where that is
+// not finite, a gradient was not (0 * inf in a row's other products would leave a NaN
+// in place of an infinity): the rows whose gradient is not finite are summed from their
+// own dot products, as the definition has them.
+__global__ __launch_bounds__(256) void ste_dmag_kernel(SteArgs g, const int8_t* __restrict__ q,
+                                                       int parts, float* __restrict__ dmag) {
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (j >= g.N) return;
+    float s = 0.0f;
+#pragma unroll 8
+    for (int c = 0; c < parts; ++c) s = __fadd_rn(s, g.part_mag[(int64_t)c * g.N + j]);
+    s = __fmul_rn(s, g.ws);
+    if (!(fabsf(s) < __builtin_inff())) {
+        float odd = 0.0f;
+        for (int i = 0; i < g.M; ++i) {
+            const float gr = g.grad[(int64_t)i * g.N + j];
+            if (fabsf(gr) < __builtin_inff()) continue;
+            int acc = 0;
+            for (int k = 0; k < g.K; ++k) {
+                const uint32_t c = (g.packed[((int64_t)j * g.K + k) >> 4] >> (2 * (k & 15))) & 3u;
+                acc += (c == 0u ? -1 : (c == 2u ? 1 : 0)) * q[(int64_t)i * g.K + k];
+            }
+            odd += gr * (static_cast<float>(acc) * (g.as[i] * g.ws));
+        }
+        if (odd != 0.0f) s = odd;  // (only finite gradients: their sum overflowed, s stands)
+    }
+    dmag[j] = s;
+}
+
+// The exact operands, reduction-contiguous in bf16: qT[k][i] = q[i][k] and tT[k][j] =
+// T[j][k], zero in the padding columns up to a multiple of 32.  A thread takes 16 k of
+// 8 rows and writes, per k, its 8 rows as 16 bytes (a k row's 64 columns of a workgroup
+// are one 128-byte line).
+__global__ __launch_bounds__(256) void ste_pack_kernel(const int8_t* __restrict__ q,
+                                                       const uint32_t* __restrict__ packed, int M,
+                                                       int K, int N, int Mp, int Np,
+                                                       uint16_t* __restrict__ qT,
+                                                       uint16_t* __restrict__ tT, int qblocks) {
+    const bool codes = (int)blockIdx.x < qblocks;
+    const int r0 = ((codes ? blockIdx.x : blockIdx.x - qblocks) * 8 + (threadIdx.x & 7)) * 8;
+    const int k0 = (blockIdx.y * 32 + (threadIdx.x >> 3)) * 16;
+    const int rows = codes ? M : N, pad = codes ? Mp : Np;
+    if (k0 >= K || r0 >= pad) return;  // pad % 8 == 0, K % 16 == 0
+    uint16_t v[16][8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        const bool in = r0 + r < rows;
+        if (codes) {
+            uint4 w = make_uint4(0u, 0u, 0u, 0u);
+            if (in) w = *reinterpret_cast<const uint4*>(q + (int64_t)(r0 + r) * K + k0);
+            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+                v[k][r] = f32_to_bf16(static_cast<float>(
+                    static_cast<int8_t>((ws[k >> 2] >> (8 * (k & 3))) & 0xffu)));
+        } else {
+            const uint32_t w = in ? packed[((int64_t)(r0 + r) * K + k0) >> 4] : 0x55555555u;
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const uint32_t c = (w >> (2 * k)) & 3u;
+                v[k][r] = c == 0u ? 0xBF80u : (c == 2u ? 0x3F80u : 0u);  // -1 / +1 / 0
+            }
+        }
+    }
+    uint16_t* dst = codes ? qT : tT;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        uint32_t w[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) w[p] = v[k][2 * p] | ((uint32_t)v[k][2 * p + 1] << 16);
+        *reinterpret_cast<uint4*>(dst + (int64_t)(k0 + k) * pad + r0) =
+            make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
+// Tensor::rmsnorm_backward (src/tensor.cpp:3997-4056) with x_norm = x * inv:
+// dot = sum_k g*y / K; dx = (g - y*dot) * inv.  One wave per row.
+template <int XDT>
+__global__ __launch_bounds__(256) void rms_backward_kernel(const void* __restrict__ x,
+                                                           const float* __restrict__ inv,
+                                                           const float* __restrict__ g, int M,
+                                                           int K, float* __restrict__ dx) {
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= M) return;
+    const float s = inv[row];
+    const int64_t base = (int64_t)row * K;
+    float dot = 0.0f;
+    for (int k = lane; k < K; k += 64) {
+        const float yv = __fmul_rn(load_act<XDT>(x, base + k), s);
+        dot = __fmaf_rn(g[base + k], yv, dot);
+    }
+    for (int off = 32; off > 0; off >>= 1) dot = __fadd_rn(dot, __shfl_xor(dot, off));
+    dot = __fdiv_rn(dot, static_cast<float>(K));
+    for (int k = lane; k < K; k += 64) {
+        const float yv = __fmul_rn(load_act<XDT>(x, base + k), s);
+        dx[base + k] = __fmul_rn(__fmaf_rn(-yv, dot, g[base + k]), s);
+    }
+}
+
+static int64_t round256(int64_t v) { return (v + 255) & ~int64_t(255); }
+
+// Row pitch of the transposed operands: whole 256-byte units, an odd number of them, so
+// that a tile's 256 rows (64 bytes of each per stage) spread over the L2 channels; a
+// power-of-two pitch puts them all on one.
+static int ste_pitch(int n) { return (n + kTK - 1) / kTK * kTK; }
+
+struct SteWorkspace {
+    uint16_t* qT;     // bf16 [K, Mp]
+    uint16_t* tT;     // bf16 [K, Np]
+    float* dact;      // [M, K] (rms_input only)
+    float* inv;       // [M] (rms_input only)
+    float* part;      // [4 * K tiles, N]
+    int Mp, Np;
+    int64_t bytes;
+};
+
+static SteWorkspace ste_layout(void* base, int M, int K, int N, int rms_input) {
+    SteWorkspace w{};
+    w.Mp = ste_pitch(M);
+    w.Np = ste_pitch(N);
+    int64_t off = 0;
+    auto take = [&](int64_t bytes) {
+        char* p = base ? static_cast<char*>(base) + off : nullptr;
+        off += round256(bytes);
+        return p;
+    };
+    w.qT = reinterpret_cast<uint16_t*>(take(2 * (int64_t)K * w.Mp));
+    w.tT = reinterpret_cast<uint16_t*>(take(2 * (int64_t)K * w.Np));
+    w.dact = rms_input ? reinterpret_cast<float*>(take(4 * (int64_t)M * K)) : nullptr;
+    w.inv = rms_input ? reinterpret_cast<float*>(take(4 * (int64_t)M)) : nullptr;
+    w.part = reinterpret_cast<float*>(take(16 * (int64_t)((K + kTC - 1) / kTC) * N));
+    w.bytes = off;
+    return w;
+}
+
+}  // namespace nsosx
+
+using namespace nsosx;
+
+extern "C" int64_t nsosx_bitlinear_ste_backward_workspace(int M, int K, int N, int rms_input) {
+    if (M <= 0 || K <= 0 || N <= 0) return 0;
+    return ste_layout(nullptr, M, K, N, rms_input).bytes;
+}
+
+extern "C" int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const int8_t* q,
+                                            const float* act_scale, const float* w_latent,
+                                            const uint32_t* packed, float weight_scale, int M,
+                                            int K, int N, int rms_input, const float* magnitude,
+                                            const float* grad, float* dx, float* dW, float* dmag,
+                                            float* dbias, void* workspace, void* stream) {
+    if (!q || !act_scale || !w_latent || !packed || !grad || !dx || !dW || !workspace)
+        return fail(NSOSX_ERR_INVALID, "bitlinear_ste_backward: null pointer");
+    if (rms_input && !x)
+        return fail(NSOSX_ERR_INVALID, "bitlinear_ste_backward: rms_input needs the input x");
+    if (dmag && !magnitude)
+        return fail(NSOSX_ERR_INVALID, "bitlinear_ste_backward: dmag needs the magnitude");
+    if (M <= 0 || K <= 0 || N <= 0)
+        return fail(NSOSX_ERR_INVALID, "bitlinear_ste_backward: empty shape");
+    if (K % 16 != 0 || N % 4 != 0)
+        return fail(NSOSX_ERR_INVALID,
+                    "bitlinear_ste_backward: K must be a multiple of 16 and N of 4");
+    if (!valid_dtype(x_dtype)) return fail(NSOSX_ERR_INVALID, "bitlinear_ste_backward: bad dtype");
+    if (!(weight_scale > 0.0f) || !std::isfinite(weight_scale))
+        return fail(NSOSX_ERR_INVALID, "bitlinear_ste_backward: weight_scale must be finite > 0");
+    if ((int64_t)M * K > ((int64_t)1 << 40) || (int64_t)M * N > ((int64_t)1 << 40) ||
+        (int64_t)N * K > ((int64_t)1 << 40))
+        return fail(NSOSX_ERR_OVERFLOW, "bitlinear_ste_backward: size too large");
+    if (reinterpret_cast<uintptr_t>(q) % 16 || reinterpret_cast<uintptr_t>(grad) % 16 ||
+        reinterpret_cast<uintptr_t>(workspace) % 256)
+        return fail(NSOSX_ERR_INVALID,
+                    "bitlinear_ste_backward: q and grad 16-byte, workspace 256-byte aligned");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const SteWorkspace ws = ste_layout(workspace, M, K, N, rms_input);
+    const int tk = (K + kTC - 1) / kTC;
+    const int64_t tiles = ((int64_t)(M + kTR - 1) / kTR + (N + kTR - 1) / kTR) * tk;
+    const int qblocks = (ws.Mp + 63) / 64, tblocks = (ws.Np + 63) / 64;
+    if (tiles > 0x7fffffff || K > 65535 * 512)
+        return fail(NSOSX_ERR_OVERFLOW, "bitlinear_ste_backward: size too large");
+
+    hipLaunchKernelGGL(ste_pack_kernel, dim3(qblocks + tblocks, (K + 511) / 512), dim3(256), 0, st,
+                       q, packed, M, K, N, ws.Mp, ws.Np, ws.qT, ws.tT, qblocks);
+    // dW = gp^T @ (x_q * act_scale), zero where |W / (ws + 1e-8f)| > 1 (bitlinear.cpp:1293-1321),
+    // with gp = grad * magnitude taken as magnitude[j] * (grad^T @ ...); d_act = gp @ (ternary *
+    // weight_scale) (1340); the column sums behind dmag and dbias (1267-1290) on the way
+    SteArgs g{};
+    g.grad = grad; g.mag = magnitude; g.as = act_scale; g.qT = ws.qT; g.tT = ws.tT;
+    g.packed = packed; g.wlat = w_latent; g.dW = dW; g.dact = rms_input ? ws.dact : dx;
+    g.part_mag = dmag ? ws.part : nullptr; g.dbias = dbias;
+    g.ws = weight_scale; g.clip = weight_scale + 1e-8f;
+    g.M = M; g.K = K; g.N = N; g.Mp = ws.Mp; g.Np = ws.Np;
+    hipLaunchKernelGGL(ste_gemm_kernel, dim3((unsigned)tiles), dim3(kSteThreads), kSteSmem, st, g);
+    if (dmag)
+        hipLaunchKernelGGL(ste_dmag_kernel, dim3((N + 255) / 256), dim3(256), 0, st, g, q, 4 * tk,
+                           dmag);
+
+    // dx = rmsnorm_backward(x, d_act, x_norm) (bitlinear.cpp:1352-1355)
+    if (rms_input) {
+        launch_rms_inv(x, x_dtype, M, K, 1e-6f, ws.inv, st);
+        const dim3 grid((M + 3) / 4);
+        if (x_dtype == NSOSX_F32)
+            hipLaunchKernelGGL((rms_backward_kernel<NSOSX_F32>), grid, dim3(256), 0, st, x, ws.inv,
+                               ws.dact, M, K, dx);
+        else
+            hipLaunchKernelGGL((rms_backward_kernel<NSOSX_BF16>), grid, dim3(256), 0, st, x,
+                               ws.inv, ws.dact, M, K, dx);
+    }
+    return check_launch("bitlinear_ste_backward");
+}

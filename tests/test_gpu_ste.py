@@ -1,0 +1,86 @@
+"""The straight-through backward's split contractions against float64 on the same codes, at the
+edges of their tiles (128 x 256 outputs, 32-deep stages) and with gradients that are not finite.
+
+Each bf16 piece's product with a code is exact, so only the float sums round: n products added
+in any order stay within n * 2^-24 of the sum of their magnitudes (plus the last scaling's two
+roundings and the gradient's own, 4 * 2^-24)."""
+import numpy as np
+import pytest
+import torch
+
+from reimagined_amd import ops
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -24
+
+
+def _case(dev, m, k, n, with_mag, seed, spread=1.0):
+    rng = np.random.default_rng(seed)
+    w = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    packed, ws = ops.pack_ternary(w)
+    codes = ops.unpack_ternary(packed, n * k).reshape(n, k).astype(np.float64)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(dev)
+    q, s = ops.quantize_activations_bitnet(x, 8)
+    grad = (rng.standard_normal((m, n)) * spread ** rng.uniform(-1, 1, (m, n))).astype(np.float32)
+    mag = rng.uniform(0.5, 1.5, n).astype(np.float32) if with_mag else None
+    return w, packed, np.float32(ws), codes, x, q, s, grad, mag
+
+
+def _run(dev, c, want_dbias=True):
+    w, packed, ws, _, x, q, s, grad, mag = c
+    t = lambda a: None if a is None else torch.from_numpy(a).to(dev)
+    got = ops.bitlinear_ste_backward(x, q, s, t(w), t(packed.view(np.int32)), float(ws), t(grad),
+                                     False, t(mag), want_dbias)
+    return {key: v.cpu().numpy() for key, v in got.items()}
+
+
+def _want(c):
+    w, _, ws, codes, _, q, s, grad, mag = c
+    q, s = q.cpu().numpy().astype(np.float64), s.cpu().numpy().astype(np.float64)
+    g = grad.astype(np.float64)
+    gp = g if mag is None else g * mag
+    keep = np.abs(w / np.float32(ws + np.float32(1e-8))) <= 1.0
+    with np.errstate(invalid="ignore"):
+        pre = (q @ codes.T) * (s * float(ws))[:, None]
+        out = {"dW": (gp.T @ (q * s[:, None])), "dx": gp @ (codes * float(ws)),
+               "dmag": (g * pre).sum(0), "dbias": g.sum(0)}
+    out["dW"] = np.where(keep, out["dW"], 0.0)
+    return out
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 16, 4), (31, 16, 36), (32, 256, 128), (33, 272, 132),
+                                   (64, 240, 124), (96, 528, 260), (129, 512, 64), (200, 1040, 384)])
+@pytest.mark.parametrize("with_mag", [True, False])
+def test_ste_sums_within_float_sum_bound(dev, m, k, n, with_mag):
+    """Gradients over twelve binades either way, so that the small pieces count."""
+    c = _case(dev, m, k, n, with_mag, 7 * m + k + n, spread=4096.0)
+    got, want = _run(dev, c), _want(c)
+    _, _, ws, codes, _, q, s, grad, mag = c
+    absw = list(c)
+    absw[7], absw[3] = np.abs(grad), np.abs(codes)
+    absw[5] = q.abs()
+    absw[0] = np.zeros_like(c[0])  # no clip
+    size = _want(tuple(absw))
+    terms = {"dW": m + 4, "dx": n + 4, "dmag": m + k + 8, "dbias": m}
+    if with_mag:
+        # dmag adds T * (sum over rows of grad * as * q): its terms' magnitudes are those of
+        # sum_k |T| sum_i |grad| as |q|
+        a = np.abs(q.cpu().numpy().astype(np.float64)) * s.cpu().numpy().astype(np.float64)[:, None]
+        size["dmag"] = float(ws) * ((np.abs(grad).astype(np.float64).T @ a) * np.abs(codes)).sum(1)
+    for key, g in got.items():
+        err = np.abs(g.astype(np.float64) - want[key])
+        assert np.all(err <= terms[key] * U * size[key] + 1e-37), key
+
+
+@pytest.mark.parametrize("m,n", [(70, 40), (64, 132)])
+def test_ste_infinities_and_nan_stay_where_they_are(dev, m, n):
+    k = 272
+    c = _case(dev, m, k, n, True, m + n)
+    grad = c[7]
+    grad[3, 5], grad[40, 6], grad[m - 1, n - 1], grad[12, 9] = np.inf, -np.inf, np.inf, np.nan
+    got, want = _run(dev, c), _want(c)
+    for key, g in got.items():
+        np.testing.assert_array_equal(np.isnan(g), np.isnan(want[key]), err_msg=key)
+        inf = np.isinf(want[key])
+        np.testing.assert_array_equal(g[inf], want[key][inf].astype(np.float32), err_msg=key)
+        assert np.array_equal(np.isinf(g), inf), key
