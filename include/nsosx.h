@@ -130,10 +130,11 @@ int nsosx_quantize_act_i8(const void* x, int x_dtype, int M, int K, int bits, in
  *              then * magnitude[n], then + bias[n] (each rounded, no fma)
  * Replaces launch_bitnet_gemm / launch_bitnet_gemv_scaled /
  * launch_bitnet_apply_act_scales_kernel (include/cuda/kernels.cuh:106-110).
- * M = 1 runs the packed-weight streaming GEMV; 2 <= M <= 32 with K in
- * {1024, 2048, 4096} (ceil(M/16) * K <= 4096) the skinny MFMA kernel (one
- * decoded word feeds 16 tokens); other M <= 8 the GEMV; larger M the int8 MFMA
- * GEMM.
+ * M = 1 runs the packed-weight streaming GEMV; K % 128 == 0 and N <= 16384 the
+ * int8 MFMA GEMMs (small tiles where 256 x 128 ones would leave CUs idle);
+ * otherwise 2 <= M <= 32 with K in {1024, 2048, 4096} (ceil(M/16) * K <= 4096)
+ * the skinny MFMA kernel (one decoded word feeds 16 tokens); other M <= 8 the
+ * GEMV; larger M the int8 MFMA GEMMs.
  *   y: [M, N] f32 or bf16 (y_dtype), may be NULL when acc_out is given.
  *   acc_out: int32 [M, N] or NULL (exposes the accumulators).
  *   magnitude, bias: f32 [N] or NULL. */
@@ -142,7 +143,7 @@ int nsosx_ternary_gemm(const int8_t* q, const float* act_scale, const uint32_t* 
                        const float* bias, void* y, int y_dtype, int32_t* acc_out, void* stream);
 
 /* Same contract, forcing one kernel: path 0 = streaming GEMV (M <= 8),
- * path 1 = MFMA GEMM (any M), path 2 = skinny MFMA (2 <= M <= 32, K in
+ * path 1 = MFMA GEMMs (any M), path 2 = skinny MFMA (2 <= M <= 32, K in
  * {1024, 2048, 4096}, ceil(M/16) * K <= 4096, M * N < 2^29).  For tests and
  * measurement. */
 int nsosx_ternary_gemm_path(const int8_t* q, const float* act_scale, const uint32_t* packed,
@@ -161,8 +162,8 @@ int nsosx_pack_mfma_layout(const uint32_t* packed, int64_t n_words, uint32_t* ou
                            void* stream);
 
 /* nsosx_ternary_gemm's contract on weights in the MFMA layout above: the
- * int8 MFMA GEMM, or for decode batches the skinny path takes (2 <= M <= 32,
- * K in {1024, 2048, 4096}) the skinny MFMA kernel on the same words.
+ * int8 MFMA GEMMs, or for decode batches the skinny path takes (2 <= M <= 32,
+ * K in {1024, 2048, 4096}) on N > 16384 the skinny MFMA kernel on the same words.
  * K % 128 == 0, K <= 264208 (the layout's operands are 64 x the ternary
  * values, so 64 * 127 * K must fit int32; larger K returns
  * NSOSX_ERR_OVERFLOW).  Same results bit for bit as nsosx_ternary_gemm on the

@@ -60,9 +60,11 @@ static int check_gemm_args(const int8_t* q, const float* as, const uint32_t* pac
     return NSOSX_OK;
 }
 
-// M = 1: the VALU GEMV; 2 <= M <= 32 where the skinny MFMA path takes the
-// shape; other M <= 8: the GEMV; else the MFMA GEMM.
+// M = 1: the VALU GEMV; a matrix the caches hold (K % 128 == 0, N <= kSmallMaxN): the
+// MFMA GEMMs, whose small tiles take it; 2 <= M <= 32 where the skinny MFMA path takes
+// the shape; other M <= 8: the GEMV; else the MFMA GEMM.
 static int ternary_gemm_auto_path(int M, int K, int N) {
+    if (M > 1 && K % kG3BK == 0 && N <= kSmallMaxN) return 1;
     if (skinny_ok(M, K, N)) return 2;
     return M <= 8 ? 0 : 1;
 }
@@ -130,8 +132,8 @@ extern "C" int nsosx_ternary_gemm_mfma(const int8_t* q, const float* act_scale,
         return fail(NSOSX_ERR_OVERFLOW, "ternary_gemm_mfma: K too large for the MFMA layout's "
                                         "64x-scaled int32 sums");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (skinny_ok(M, K, N)) {
-        // decode batches: the skinny MFMA kernel on the same words
+    if (skinny_ok(M, K, N) && N > kSmallMaxN) {
+        // decode batches on a matrix past the caches: the skinny MFMA kernel on the same words
         GemvProblem pb{packed_mfma, magnitude, bias, weight_scale, N, K};
         launch_skinny(pb, q, act_scale, M, y, y_dtype, acc_out, true, st);
         return check_launch("ternary_gemm_mfma");

@@ -187,6 +187,20 @@ void launch_skinny(const GemvProblem& pb, const int8_t* q, const float* as, int 
 void launch_grouped_skinny(dim3 grid, const nsosx_linear_view* views, const int8_t* q,
                            int64_t q_stride, const float* act_scale, int64_t scale_stride, int M,
                            void* y, int64_t y_stride, int y_dtype, hipStream_t st);
+// gemm_small.hip: outputs too small for the 256 x 128 tiles (K % 128 == 0), on either layout;
+// false where those are the faster ones (nothing launched).  kSmallMaxN: up to here the
+// small tiles also beat the skinny kernel and the GEMV at 2 .. 32 rows (measured at K 1024 /
+// 2048 / 4096: 3.2 / 3.8 / 5.0 us against 3.9 / 6.0 / 9.8); on larger matrices, which stream
+// their weights from HBM, the skinny kernel's four times smaller load traffic wins.
+constexpr int kSmallMaxN = 16384;
+bool launch_gemm_small(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,
+                       int y_dtype, int32_t* acc, bool mfma_layout, hipStream_t st);
+// the experts' row segments, MFMA layout (perm null: rows already in slot order);
+// large_extra: what the tiled launch would cost besides its tiles, in 0.1 us
+bool launch_grouped_gemm_small(const nsosx_linear_view* views, int experts, const int32_t* offsets,
+                               const int32_t* perm, const int8_t* q, const float* as, int K, int N,
+                               int total_rows, int sqrelu, void* y, int y_dtype, double large_extra,
+                               hipStream_t st);
 // gemm.hip: the MFMA GEMMs on the reference words and on the MFMA layout
 void launch_gemm(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,
                  int y_dtype, int32_t* acc, hipStream_t st);

@@ -90,7 +90,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmProblem pb, const int8_t*
 template <int YDT>
 static void launch_gemm_t(const GemmProblem& pb, const int8_t* q, const float* as, int M,
                           void* y, int32_t* acc, hipStream_t st) {
-    if (M > kBM) {
+    if (launch_gemm_small(pb, q, as, M, y, YDT, acc, false, st)) return;
+    if (M > kBM || pb.K % kG3BK == 0) {
         const int tiles = ((pb.N + kBN2 - 1) / kBN2) * ((M + kBM2 - 1) / kBM2);
         if (pb.K % kG3BK == 0) {
             const int tiles3 = ((pb.N + kG3BN - 1) / kG3BN) * ((M + kG3BM - 1) / kG3BM);
@@ -125,6 +126,7 @@ void launch_gemm(const GemmProblem& pb, const int8_t* q, const float* as, int M,
 
 void launch_gemm_mfma(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,
                       int y_dtype, int32_t* acc, hipStream_t st) {
+    if (launch_gemm_small(pb, q, as, M, y, y_dtype, acc, true, st)) return;
     const int tiles = ((pb.N + kG3BN - 1) / kG3BN) * ((M + kG3BM - 1) / kG3BM);
 #define NSOSX_GM(YDT, ACC)                                                                    \
     hipLaunchKernelGGL((gemm3_mfma_kernel<YDT, ACC>), dim3(tiles), dim3(kGemm3Threads), kGemm3Smem, \

@@ -1,0 +1,87 @@
+"""The small-tile ternary GEMMs (32 / 64 outputs x 32 / 64 tokens, K split over four waves) at the
+edges of their tiles and of the rule that picks them, on both weight layouts: accumulators and
+outputs bit for bit against the integer product and the reference's affine (each step rounded)."""
+import numpy as np
+import pytest
+import torch
+
+from reimagined_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(rng, n, k):
+    codes = rng.integers(-1, 2, (n, k)).astype(np.int64)
+    words = ((codes + 1).astype(np.uint32).reshape(n * k // 16, 16) << (2 * np.arange(16, dtype=np.uint32)))
+    return codes, words.sum(1, dtype=np.uint32)
+
+
+def _affine(acc, s, ws, mag, bias):
+    v = acc.astype(np.float32) * (s * np.float32(ws))[:, None]
+    if mag is not None:
+        v = v * mag
+    return v if bias is None else v + bias
+
+
+# K of 1, 2, 3, 4, 5 and 9 blocks of 128 (waves with no block, uneven quarters); row counts and
+# widths on either side of 32 / 64; 2048 x 3 000-odd rows past the point where large tiles win
+@pytest.mark.parametrize("m,k,n", [(2, 128, 32), (9, 256, 33), (31, 384, 7), (32, 512, 64),
+                                   (33, 640, 100), (64, 1152, 129), (65, 128, 768), (100, 2048, 8192),
+                                   (300, 768, 768), (257, 1024, 4104), (700, 2048, 1000),
+                                   (3001, 2048, 520)])
+@pytest.mark.parametrize("mfma", [True, False])
+@pytest.mark.parametrize("ydt", [torch.float32, torch.bfloat16])
+def test_small_tiles_bit_exact(dev, m, k, n, mfma, ydt):
+    rng = np.random.default_rng(m + 3 * k + n)
+    codes, words = _matrix(rng, n, k)
+    q = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    s = rng.uniform(0.01, 0.1, m).astype(np.float32)
+    mag = rng.uniform(0.5, 1.5, n).astype(np.float32) if n % 2 == 0 else None
+    bias = rng.standard_normal(n).astype(np.float32) if m % 2 == 0 else None
+    t = lambda a: None if a is None else torch.from_numpy(a).to(dev)
+    packed = t(words.view(np.int32))
+    if mfma:
+        y, acc = ops.ternary_gemm_mfma(t(q), t(s), ops.pack_mfma_layout(packed), 0.37, n, t(mag),
+                                       t(bias), out_dtype=ydt, want_acc=True)
+    else:
+        y, acc = ops.ternary_gemm(t(q), t(s), packed, 0.37, n, t(mag), t(bias), out_dtype=ydt,
+                                  want_acc=True, path=1)
+    # |acc| <= 127 * 2048: exact in float64
+    want = np.rint(q.astype(np.float64) @ codes.T.astype(np.float64)).astype(np.int32)
+    np.testing.assert_array_equal(acc.cpu().numpy(), want)
+    wy = torch.from_numpy(_affine(want, s, 0.37, mag, bias)).to(ydt)
+    np.testing.assert_array_equal(y.float().cpu().numpy(), wy.float().numpy())
+
+
+@pytest.mark.parametrize("rows", [[5], [0, 1, 33, 64, 65, 0, 31, 2], [12] * 8, [0, 0, 200, 0],
+                                  [130, 7, 64, 300]])
+@pytest.mark.parametrize("k,n", [(128, 96), (1024, 520), (4096, 256)])
+@pytest.mark.parametrize("gather", [True, False])
+def test_grouped_small_tiles_bit_exact(dev, rows, k, n, gather):
+    rng = np.random.default_rng(sum(rows) + k + n)
+    slots = sum(rows)
+    mats = [_matrix(rng, n, k) for _ in rows]
+    mags = [rng.uniform(0.5, 1.5, n).astype(np.float32) for _ in rows]
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    views = ops.LinearViewArray([(ops.pack_mfma_layout(t(w.view(np.int32))), 0.3 + 0.01 * e, k, n,
+                                  t(mags[e]) if e % 2 else None, None)
+                                 for e, (_, w) in enumerate(mats)], dev)
+    offsets = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    perm = rng.permutation(slots).astype(np.int32)
+    q = rng.integers(-127, 128, (slots, k)).astype(np.int8)
+    s = rng.uniform(0.01, 0.1, slots).astype(np.float32)
+    ws = torch.empty(ops.grouped_mfma_workspace_bytes(), dtype=torch.uint8, device=dev)
+    for sq, work in ((False, None), (True, ws)):
+        y = ops.grouped_ternary_gemm_mfma(views, t(offsets), t(perm), t(q), t(s), n, slots,
+                                          squared_relu=sq, gather=gather, workspace=work)
+        want = np.empty((slots, n), np.float32)
+        for e, (codes, _) in enumerate(mats):
+            seg = np.arange(offsets[e], offsets[e + 1])
+            src = perm[seg] if gather else seg
+            acc = np.rint(q[src].astype(np.float64) @ codes.T.astype(np.float64))
+            v = _affine(acc, s[src], np.float32(0.3 + 0.01 * e), mags[e] if e % 2 else None, None)
+            if sq:
+                v = np.where(v > 0, v, np.float32(0))
+                v = v * v
+            want[seg] = v
+        np.testing.assert_array_equal(y.cpu().numpy(), want)
