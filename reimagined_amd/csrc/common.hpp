@@ -65,6 +65,25 @@ __device__ __forceinline__ float load_act(const void* p, int64_t i) {
     }
 }
 
+// 8 consecutive activations as floats (bf16 widened exactly).
+template <int DT>
+__device__ __forceinline__ void load8(const void* x, int64_t off, float v[8]) {
+    if constexpr (DT == NSOSX_F32) {
+        const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(x) + off);
+        const float4 a = p[0], b = p[1];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
+        const uint4 a = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(x) + off);
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = __uint_as_float(w[i] << 16);
+            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+        }
+    }
+}
+
 // Raw storage word of an activation element: kept unconverted in registers, a
 // prefetched value costs no wait until raw_to_f32() is applied where it is used.
 template <int DT> struct raw_word { using type = uint32_t; };

@@ -295,24 +295,6 @@ constexpr int kSkinnyRows = 32;   // rows per workgroup
 constexpr int kSkinnyMaxN = 64;
 constexpr int kSkinnyWaves = 4;   // K split
 
-template <int XDT>
-__device__ __forceinline__ void load8(const void* p, int64_t i, float v[8]) {
-    if constexpr (XDT == NSOSX_F32) {
-        const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i);
-        const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-        const u32x4 u = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p) + i);
-        const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[2 * j] = __uint_as_float(wd[j] << 16);
-            v[2 * j + 1] = __uint_as_float(wd[j] & 0xFFFF0000u);
-        }
-    }
-}
-
 template <int XDT, int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 2 : 3))) void skinny_f32_kernel(const void* __restrict__ x, int rms,
                                                      float eps, const float* __restrict__ w, int M,

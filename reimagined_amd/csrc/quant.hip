@@ -5,6 +5,7 @@
 //   quantization  src/bitlinear.cpp:240-291, src/bitlinear_quantize_avx2.cpp:65-103
 //   RMS_PERI norm src/bitlinear.cpp:460-466, src/tensor.cpp:3455-3492
 #include "bitlinear.hpp"
+#include "row_sum.hpp"
 
 namespace nsosx {
 
@@ -292,17 +293,70 @@ __global__ __launch_bounds__(256) void rms_inv_small_kernel(const void* __restri
 // (load8 and the one-row quantize_row_wg live in bitlinear.hpp: the decode
 // projections of gemv.hip use them too.)
 // ===========================================================================
+// ===========================================================================
+// RMS_PERI + codes in one launch, a workgroup per row (row_sum.hpp takes the in-order sum;
+// by one lane walking the row from LDS it was 4.2 us of a call at K = 1024 and 16 us at 4096).
+// The absmax of x * inv is round(max|x| * inv): rounding is monotonic.
+// Time per call, us, before (a serial sum up to 1024 rows, two passes above) -> now:
+//   bf16   1 x 1024 6.4 -> 5.0    64 x 2048 11.4 -> 6.4    1024 x 4096 32.8 -> 11.6
+//   f32  300 x 768  6.8 -> 5.7  1500 x 2048 18.2 -> 9.6    3000 x 4096 38.8 -> 27.4
+// It is bound by instruction issue (about 1000 per 1024-element row, half of them the walk),
+// so past 3072 rows of bf16 the two streaming passes, a lane per row, are the faster ones
+// (4096 x 2048: 17.2 against 18.5 us), and past 6144 rows of f32 (4096 where K < 1024).
+// ===========================================================================
 template <int DT>
-__global__ __launch_bounds__(256) void quantize_small_rms_kernel(const void* __restrict__ x,
-                                                                 int K, float q_max, float eps,
-                                                                 float* __restrict__ rms_inv,
-                                                                 int8_t* __restrict__ q,
-                                                                 float* __restrict__ act_scale) {
-    __shared__ __align__(16) float s_row[kQSmallMaxK];
-    __shared__ float s_red[5];
-    const int row = blockIdx.x;
-    quantize_row_wg<DT, true>(x, (int64_t)row * K, K, q_max, eps, s_row, s_red,
-                              q + (int64_t)row * K, act_scale + row, rms_inv + row);
+__global__ __launch_bounds__(512) void quantize_row_rms_kernel(const void* __restrict__ x, int K,
+                                                               float q_max, float eps,
+                                                               float* __restrict__ rms_inv,
+                                                               int8_t* __restrict__ q,
+                                                               float* __restrict__ act_scale) {
+    extern __shared__ __align__(16) float s_dyn[];  // 8 floats per thread, then a SumRun each
+    __shared__ unsigned long long s_mask[8];
+    __shared__ float s_w[8], s_max[8], s_inv;
+    float* s_sq = s_dyn;
+    SumRun* s_run = reinterpret_cast<SumRun*>(s_dyn + 8 * blockDim.x);
+    const int64_t row = blockIdx.x;
+    const int tid = threadIdx.x;
+    const bool in = tid * 8 < K;  // K % 8 == 0
+    float v[8], sq[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = 0.0f;
+    if (in) load8<DT>(x, row * K + tid * 8, v);
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        sq[j] = __fmul_rn(v[j], v[j]);
+        m = fmaxf(m, fabsf(v[j]));
+    }
+    *reinterpret_cast<float4*>(s_sq + tid * 8) = make_float4(sq[0], sq[1], sq[2], sq[3]);
+    *reinterpret_cast<float4*>(s_sq + tid * 8 + 4) = make_float4(sq[4], sq[5], sq[6], sq[7]);
+    m = wave_max(m);
+    if ((tid & 63) == 0) s_max[tid >> 6] = m;
+    // (adding the zeros past the row's end leaves the sum as it is)
+    const float sum = row_sum_in_order(sq, s_sq, s_run, s_w, s_mask);
+    if (tid == 0) {
+        const float mean = __fdiv_rn(sum, static_cast<float>(K));
+        const float inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, eps)));
+        s_inv = inv;
+        rms_inv[row] = inv;
+    }
+    __syncthreads();
+    const float inv = s_inv;
+    m = 0.0f;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = fmaxf(m, s_max[w]);
+    // an infinite x gives inf * 0, which the absmax of the products skips
+    m = fmaxf(0.0f, __fmul_rn(m, inv));
+    const float denom = __fadd_rn(m, 1e-8f);
+    const float sc = __fdiv_rn(q_max, denom);
+    if (tid == 0) act_scale[row] = __fdiv_rn(denom, q_max);
+    if (!in) return;
+    float code[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) code[j] = clamp127(rintf(__fmul_rn(__fmul_rn(v[j], inv), sc)));
+    uint2 out;
+    out.x = pack4_i8(code[0], code[1], code[2], code[3]);
+    out.y = pack4_i8(code[4], code[5], code[6], code[7]);
+    *reinterpret_cast<uint2*>(q + row * K + tid * 8) = out;
 }
 
 template <int DT, bool RMS>
@@ -536,10 +590,12 @@ static int launch_quantize(const void* x, int M, int K, int bits, int rms_input,
                            float* act_scale, float* rms_ws, hipStream_t st) {
     const float qm = q_max_for_bits(bits);
     const int elem = DT == NSOSX_F32 ? 4 : 2;
-    if (rms_input && M <= 1024 && K % 8 == 0 && K <= kQSmallMaxK &&
+    const int few = DT == NSOSX_BF16 ? 3072 : (K >= 1024 ? 6144 : 4096);
+    if (rms_input && M <= few && K % 8 == 0 && K <= kQSmallMaxK &&
         reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 8 == 0) {
-        hipLaunchKernelGGL((quantize_small_rms_kernel<DT>), dim3(M), dim3(256), 0, st, x, K, qm,
-                           1e-6f, rms_ws, q, act_scale);
+        const int threads = (K / 8 + 63) / 64 * 64;
+        hipLaunchKernelGGL((quantize_row_rms_kernel<DT>), dim3(M), dim3(threads),
+                           row_sum_smem(threads), st, x, K, qm, 1e-6f, rms_ws, q, act_scale);
         return check_launch("quantize_act");
     }
     if (rms_input) launch_rms_inv_t<DT>(x, M, K, 1e-6f, rms_ws, st);

@@ -1,0 +1,240 @@
+// The in-order float sum of a row's squares by one workgroup, without the chain of K
+// dependent adds: shared by the activation quantizer (quant.hip) and the straight-through
+// backward's row norm (ste.hip).
+//
+// Reference semantics (OXN/nsos/ of vitorGgC569/reimagined): the sequential sum of
+// Tensor::rmsnorm, src/tensor.cpp:3455-3492.
+#pragma once
+#include "common.hpp"
+
+namespace nsosx {
+
+// ===========================================================================
+// Eight consecutive elements per thread.  The in-order float sum S <- round(S + v_k) is a chain
+// of K dependent adds (one lane walking the row from LDS: 8.8 cycles each, 4.2 us at
+// K = 1024, 16 us at 4096), but inside one binade of S its rounding depends on S only
+// through S's last bit: with S = 2^e + n ulp, round(S + v) - S is the same for every even n
+// and the same for every odd n (ties go to the even neighbour).  So, the squares being >= 0,
+// a run of elements that stays inside binade e is a pair of increments in ulps (for an even
+// and an odd start), found by adding the run to 2^e and to 2^e + ulp, and runs compose:
+// (a then b) adds a_p + b_{(p + a_p) & 1}.
+//   1. every thread sums its squares; a scan gives each thread an estimate of S at its
+//      first element, hence the binade it expects, and the element (if any) at which S
+//      enters another one;
+//   2. each thread runs the two additions over its eight elements, before (A) and after (B)
+//      that element; a segmented scan composes the increments of neighbouring threads;
+//   3. one wave walks the row's segments (about log2 K of them) with the true S in scalar
+//      registers: an increment per run, one real float add per crossing.  The estimate
+//      is never trusted: a run counts only if S starts and ends in the expected binade,
+//      else (and at the row's start, at zeros, infinities and NaN, or where one thread's
+//      elements cross twice) its elements are added one by one.  Same sum bit for bit.
+// ===========================================================================
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp0(int v) {  // 0 where the lane has no source
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143, kDppWaveShr1 = 0x138;
+
+// one thread's part of the row for the walk
+struct SumRun {
+    int d0, d1;  // composed increments of the segment up to this thread (B if it crosses)
+    int r0, r1;  // this thread's own (B)
+    int a0, a1;  // increments before its crossing element
+    float v;     // the crossing element
+    int meta;    // binade of d (8 bits), binade of a (8), index of the element (4), kind
+};
+constexpr int kSumCross = 1 << 20, kSumSerial = 2 << 20;
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void sum_scan_step(int& d0, int& d1, int& head) {
+    const int p0 = dpp0<CTRL, ROWS>(d0), p1 = dpp0<CTRL, ROWS>(d1), ph = dpp0<CTRL, ROWS>(head);
+    const int n0 = p0 + ((p0 & 1) ? d1 : d0);
+    const int n1 = p1 + ((p1 & 1) ? d0 : d1);
+    d0 = head ? d0 : n0;
+    d1 = head ? d1 : n1;
+    head |= ph;
+}
+
+__device__ __forceinline__ void sum_scan(int& d0, int& d1, int head) {
+    sum_scan_step<kDppShr1, 0xF>(d0, d1, head);
+    sum_scan_step<kDppShr2, 0xF>(d0, d1, head);
+    sum_scan_step<kDppShr4, 0xF>(d0, d1, head);
+    sum_scan_step<kDppShr8, 0xF>(d0, d1, head);
+    sum_scan_step<kDppBcast15, 0xA>(d0, d1, head);
+    sum_scan_step<kDppBcast31, 0xC>(d0, d1, head);
+}
+
+__device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+
+// The in-order sum of the row's squares, in s_sq (thread t's: sq) with K = 8 * blockDim.x
+// entries, zeros past the row's end; returned to wave 0.  s_run: blockDim.x entries; s_w: 8
+// floats and 8 masks.
+__device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const float* s_sq,
+                                                  SumRun* s_run, float* s_w,
+                                                  unsigned long long* s_mask) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const float own = ((sq[0] + sq[1]) + (sq[2] + sq[3])) + ((sq[4] + sq[5]) + (sq[6] + sq[7]));
+    float incl = own;
+    incl += __int_as_float(dpp0<kDppShr1>(__float_as_int(incl)));
+    incl += __int_as_float(dpp0<kDppShr2>(__float_as_int(incl)));
+    incl += __int_as_float(dpp0<kDppShr4>(__float_as_int(incl)));
+    incl += __int_as_float(dpp0<kDppShr8>(__float_as_int(incl)));
+    incl += __int_as_float(dpp0<kDppBcast15, 0xA>(__float_as_int(incl)));
+    incl += __int_as_float(dpp0<kDppBcast31, 0xC>(__float_as_int(incl)));
+    if (lane == 63) s_w[wave] = incl;
+    __syncthreads();  // s_sq and the waves' sums
+    float r = __int_as_float(dpp0<kDppWaveShr1>(__float_as_int(incl)));
+    for (int w = 0; w < wave; ++w) r += s_w[w];
+
+    const uint32_t kExp = 0x7f800000u;
+    SumRun run;
+    run.a0 = run.a1 = 0;
+    run.v = 0.0f;
+    const uint32_t ea = __float_as_uint(r) & kExp;
+    float t0 = __uint_as_float(ea), t1 = __uint_as_float(ea | 1u);
+    int crossings = 0, at = 0;
+    uint32_t eb = ea;
+    if (__ballot((__float_as_uint(r + own) & kExp) != ea) == 0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            t0 = __fadd_rn(t0, sq[i]);
+            t1 = __fadd_rn(t1, sq[i]);
+        }
+    } else {
+        float c0 = t0, c1 = t1;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            r = __fadd_rn(r, sq[i]);
+            const uint32_t en = __float_as_uint(r) & kExp;
+            const bool cross = en != eb;
+            const float n0 = __fadd_rn(t0, sq[i]), n1 = __fadd_rn(t1, sq[i]);
+            c0 = cross ? t0 : c0;
+            c1 = cross ? t1 : c1;
+            run.v = cross ? sq[i] : run.v;
+            at = cross ? i : at;
+            crossings += cross ? 1 : 0;
+            t0 = cross ? __uint_as_float(en) : n0;
+            t1 = cross ? __uint_as_float(en | 1u) : n1;
+            eb = en;
+        }
+        if (crossings) {
+            run.a0 = (int)(__float_as_uint(c0) - ea);
+            run.a1 = (int)(__float_as_uint(c1) - (ea | 1u));
+        }
+    }
+    run.d0 = (int)(__float_as_uint(t0) - eb);
+    run.d1 = (int)(__float_as_uint(t1) - (eb | 1u));
+    // threads whose elements are added one by one: a start at zero (or a denormal), a binade with no successor, two crossings,
+    // or an estimate that disagrees with the thread before
+    const uint32_t before = (uint32_t)dpp0<kDppWaveShr1>((int)eb);
+    const bool serial = ea == 0u || eb >= (0xfeu << 23) || crossings > 1 || (lane > 0 && before != ea);
+    if (serial) run.d0 = run.d1 = 0;
+    run.r0 = run.d0;
+    run.r1 = run.d1;
+    int head = serial || crossings == 1;
+    run.meta = (int)(eb >> 23) | (int)(ea >> 23) << 8 | at << 16 |
+               (serial ? kSumSerial : (crossings == 1 ? kSumCross : 0));
+    const unsigned long long heads = __ballot(head);
+    sum_scan(run.d0, run.d1, head);
+    if (wave > 0) s_run[threadIdx.x] = run;
+    if (lane == 0) s_mask[wave] = heads;
+    __syncthreads();
+    if (wave > 0) return 0.0f;
+
+    uint32_t s = 0;  // S's bits
+    int pos = 0;     // elements added
+    auto one_by_one = [&](int end) {  // at most to the end of pos's thread
+        const float4 a = *reinterpret_cast<const float4*>(s_sq + (pos & ~7));
+        const float4 b = *reinterpret_cast<const float4*>(s_sq + (pos & ~7) + 4);
+        const float c[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const int lo = pos & 7, hi = end - (pos & ~7);
+        float f = __uint_as_float(s);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float n = __fadd_rn(f, c[i]);
+            f = i >= lo && i < hi ? n : f;
+        }
+        s = (uint32_t)__builtin_amdgcn_readfirstlane(__float_as_int(f));
+        pos = end;
+    };
+    for (int w = 0; w < waves; ++w) {
+        const SumRun cur = run;
+        if (w + 1 < waves) run = s_run[(w + 1) * 64 + lane];
+        const uint32_t mlo = __builtin_amdgcn_readfirstlane((int)s_mask[w]);
+        const uint32_t mhi = __builtin_amdgcn_readfirstlane((int)(s_mask[w] >> 32));
+        unsigned long long mask = (unsigned long long)mhi << 32 | mlo;
+        const int first = w * 64;
+        // the run of threads [from, to) of this wave, composed from its head
+        auto advance = [&](int from, int to) {
+            const uint32_t e = (uint32_t)read_lane(cur.meta, to - 1) & 0xffu;
+            const uint32_t whole = s + (uint32_t)((s & 1u) ? read_lane(cur.d1, to - 1)
+                                                           : read_lane(cur.d0, to - 1));
+            if ((s >> 23) == e && (whole >> 23) == e) {
+                s = whole;
+                pos = (first + to) * 8;
+                return;
+            }
+            int d0 = cur.d0, d1 = cur.d1;
+            for (;;) {
+                if ((s >> 23) == e) {
+                    const uint32_t n = s + (uint32_t)((s & 1u) ? d1 : d0);  // after each thread
+                    unsigned long long out = __ballot((n >> 23) != e) & (~0ull << from);
+                    if (to < 64) out &= (1ull << to) - 1;
+                    const int f = out ? __builtin_ctzll(out) : to;
+                    if (f > from) {
+                        s = (uint32_t)read_lane((int)n, f - 1);
+                        pos = (first + f) * 8;
+                    }
+                    if (f == to) return;
+                    from = f;
+                }
+                // S is not where it was expected (a crossing an element early or late): this
+                // thread's elements one by one, then the run from the next thread on
+                one_by_one((first + from + 1) * 8);
+                if (++from == to) return;
+                if ((s >> 23) == e) {
+                    d0 = cur.r0;
+                    d1 = cur.r1;
+                    sum_scan(d0, d1, lane == from);
+                }
+            }
+        };
+        int from = 0;
+        for (;;) {
+            const int next = mask ? __builtin_ctzll(mask) : 64;
+            if (pos < (first + next) * 8) advance(from, next);
+            if (next == 64) break;
+            mask &= mask - 1;
+            const int meta = read_lane(cur.meta, next);
+            const int at_el = (first + next) * 8;
+            if (meta & kSumSerial) {
+                one_by_one(at_el + 8);
+                from = next + 1;
+            } else {
+                const int j = at_el + ((meta >> 16) & 15);
+                const uint32_t n = s + (uint32_t)((s & 1u) ? read_lane(cur.a1, next) : read_lane(cur.a0, next));
+                const uint32_t e = (uint32_t)(meta >> 8) & 0xffu;
+                if ((s >> 23) == e && (n >> 23) == e) {
+                    const float v = __int_as_float(read_lane(__float_as_int(cur.v), next));
+                    s = (uint32_t)__builtin_amdgcn_readfirstlane(
+                        __float_as_int(__fadd_rn(__uint_as_float(n), v)));
+                    pos = j + 1;
+                } else {
+                    one_by_one(j + 1);
+                }
+                from = next;  // its B is the head of the next run
+            }
+        }
+    }
+    return __uint_as_float(s);
+}
+
+// LDS bytes of the row kernels: the squares and a SumRun per thread.
+inline unsigned row_sum_smem(int threads) {
+    return threads * (8 * sizeof(float) + sizeof(SumRun));
+}
+
+}  // namespace nsosx

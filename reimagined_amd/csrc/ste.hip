@@ -12,7 +12,7 @@
 // launch of 213 us for both contractions and the column sums (MFMA issue alone: 94 us at
 // the ~2.1 GHz it runs at; dW's strided gradient reads and its epilogue make its tiles the
 // longer ones), a forward and backward step 1061 -> 267 us.
-#include "common.hpp"
+#include "row_sum.hpp"
 
 #include <cmath>
 
@@ -484,6 +484,56 @@ __global__ __launch_bounds__(256) void rms_backward_kernel(const void* __restric
     }
 }
 
+// The same for rows of up to 4096 elements (K % 8 == 0), with the row's RMS on the way: a
+// workgroup per row, eight elements per thread, x and the gradient read once (the two
+// launches, which read x twice and the gradient twice: 9 + 20 us at 4096 x 1024).
+template <int XDT>
+__global__ __launch_bounds__(512) void rms_backward_row_kernel(const void* __restrict__ x, float eps,
+                                                               const float* __restrict__ g, int K,
+                                                               float* __restrict__ dx) {
+    extern __shared__ __align__(16) float s_dyn[];
+    __shared__ unsigned long long s_mask[8];
+    __shared__ float s_w[8], s_dot[8], s_inv;
+    const int64_t base = (int64_t)blockIdx.x * K;
+    const int tid = threadIdx.x;
+    const bool in = tid * 8 < K;
+    float v[8], sq[8], gr[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = gr[j] = 0.0f;
+    if (in) {
+        load8<XDT>(x, base + tid * 8, v);
+        load8<NSOSX_F32>(g, base + tid * 8, gr);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sq[j] = __fmul_rn(v[j], v[j]);
+    *reinterpret_cast<float4*>(s_dyn + tid * 8) = make_float4(sq[0], sq[1], sq[2], sq[3]);
+    *reinterpret_cast<float4*>(s_dyn + tid * 8 + 4) = make_float4(sq[4], sq[5], sq[6], sq[7]);
+    const float sum = row_sum_in_order(sq, s_dyn, reinterpret_cast<SumRun*>(s_dyn + 8 * blockDim.x),
+                                       s_w, s_mask);
+    if (tid == 0)
+        s_inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, static_cast<float>(K)), eps)));
+    __syncthreads();
+    const float s = s_inv;
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        v[j] = __fmul_rn(v[j], s);
+        dot = __fmaf_rn(gr[j], v[j], dot);
+    }
+    dot = wave_sum(dot);
+    if ((tid & 63) == 0) s_dot[tid >> 6] = dot;
+    __syncthreads();
+    dot = 0.0f;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) dot += s_dot[w];
+    dot = __fdiv_rn(dot, static_cast<float>(K));
+    if (!in) return;
+    float o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = __fmul_rn(__fmaf_rn(-v[j], dot, gr[j]), s);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dx[base + tid * 8 + j] = o[j];
+}
+
 static int64_t round256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
 // Row pitch of the transposed operands: whole 256-byte units, an odd number of them, so
@@ -582,6 +632,16 @@ extern "C" int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const in
 
     // dx = rmsnorm_backward(x, d_act, x_norm) (bitlinear.cpp:1352-1355)
     if (rms_input) {
+        if (K <= 4096 && reinterpret_cast<uintptr_t>(x) % 16 == 0) {  // K % 16 == 0: whole chunks
+            const int threads = (K / 8 + 63) / 64 * 64;
+            if (x_dtype == NSOSX_F32)
+                hipLaunchKernelGGL((rms_backward_row_kernel<NSOSX_F32>), dim3(M), dim3(threads),
+                                   row_sum_smem(threads), st, x, 1e-6f, ws.dact, K, dx);
+            else
+                hipLaunchKernelGGL((rms_backward_row_kernel<NSOSX_BF16>), dim3(M), dim3(threads),
+                                   row_sum_smem(threads), st, x, 1e-6f, ws.dact, K, dx);
+            return check_launch("bitlinear_ste_backward");
+        }
         launch_rms_inv(x, x_dtype, M, K, 1e-6f, ws.inv, st);
         const dim3 grid((M + 3) / 4);
         if (x_dtype == NSOSX_F32)

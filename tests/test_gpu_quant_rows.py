@@ -1,0 +1,67 @@
+"""RMS_PERI + int8 codes of few rows (a workgroup per row, the in-order sum taken from composed
+runs): codes and scales bit for bit against the oracle's sequential sum, on rows built to hit the
+runs' edges -- ties at every addition, sums that sit on a binade's end, jumps over several
+binades, zeros, denormals, and values that are not finite."""
+import numpy as np
+import pytest
+import torch
+
+from reimagined_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(rng, k, bf16):
+    n = lambda *s: rng.standard_normal(s if s else k)
+    rows = [n(), n() * 1e-3, np.ones(k), np.full(k, 2.0 ** -12), np.full(k, 3.0 * 2.0 ** -13)]
+    # heavy tails: the sum jumps binades at random places
+    rows += [np.exp(4.0 * n()) * np.sign(n()), rng.standard_cauchy(k)]
+    # squares that are exact halves of an ulp of the sum from the second element on
+    tie = np.full(k, 2.0 ** -12); tie[0] = 1.0
+    rows.append(tie)
+    tie = np.full(k, 2.0 ** -12 * 1.5); tie[0] = 1.0
+    rows.append(tie)
+    # the sum stands just below a power of two, then crosses by one ulp at the row's end
+    edge = np.zeros(k); edge[0] = np.sqrt(1.0 - 2.0 ** -20); edge[1:] = 2.0 ** -13
+    rows.append(edge)
+    up = np.zeros(k); up[k // 2:] = 1.0
+    rows.append(up)
+    rows.append(np.zeros(k))
+    jump = np.full(k, 2.0 ** -10); jump[k // 3] = 300.0; jump[-1] = 1e4
+    rows.append(jump)
+    rows.append(np.full(k, 1e-22))                       # denormal squares and sums
+    rows.append(np.where(np.arange(k) % 7 == 0, 1e-3, 1e-22))
+    rows.append(np.exp2(np.linspace(-40, 40, k)))        # a crossing every few elements
+    rows.append(np.exp2(np.linspace(40, -40, k)))
+    rows.append(n() * 1e18)                              # sums near the top of the range
+    rows += [n() * (0.5 + 0.1 * i) for i in range(15)]
+    x = np.stack(rows).astype(np.float32)
+    return torch.from_numpy(x).to(torch.bfloat16).float().numpy() if bf16 else x
+
+
+@pytest.mark.parametrize("k", [8, 16, 64, 504, 512, 520, 768, 1024, 1032, 2048, 2560, 4088, 4096])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_few_rows_rms_codes_bit_exact(dev, orc, k, bf16):
+    x = _rows(np.random.default_rng(k), k, bf16)
+    xd = torch.from_numpy(x).to(torch.bfloat16 if bf16 else torch.float32).to(dev)
+    q, s = ops.quantize_activations_bitnet(xd, 8, rms_input=True)
+    wq, ws = orc.quantize_act(orc.rmsnorm(x), 8)
+    np.testing.assert_array_equal(s.cpu().numpy(), ws)
+    np.testing.assert_array_equal(q.cpu().numpy(), wq)
+
+
+@pytest.mark.parametrize("k", [512, 1024, 4096])
+def test_few_rows_equal_many_rows(dev, k):
+    """The same rows through this launch and through the passes that take many rows, also with
+    infinities and NaN (whose codes and scales both define as the arithmetic falls)."""
+    rng = np.random.default_rng(k + 1)
+    x = rng.standard_normal((64, k)).astype(np.float32)
+    x[3, 5], x[4, k - 1], x[5, 0], x[6, 7] = np.inf, -np.inf, np.nan, 3e38
+    x[7] = np.inf
+    x[8, :9] = [np.inf, np.nan, 0, 0, 1, 1, 1, 1, np.inf]
+    few = torch.from_numpy(x).to(dev)
+    q, s = ops.quantize_activations_bitnet(few, 8, rms_input=True)
+    many = torch.cat([few, torch.ones((40000, k), device=dev)])
+    wq, ws = ops.quantize_activations_bitnet(many, 8, rms_input=True)
+    np.testing.assert_array_equal(q.cpu().numpy(), wq[:64].cpu().numpy())
+    np.testing.assert_array_equal(s.cpu().numpy(), ws[:64].cpu().numpy())
