@@ -103,6 +103,9 @@ extern "C" int nsosx_ternary_gemm(const int8_t* q, const float* act_scale, const
                                    y_dtype, acc_out, ternary_gemm_auto_path(M, K, N), stream);
 }
 
+// Widest layer whose one-row forward is one launch.
+constexpr int kRowMaxN = 16384;
+
 extern "C" int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_t* packed,
                                        float weight_scale, int M, int K, int N,
                                        int precision_bits, int rms_input, const float* magnitude,
@@ -113,6 +116,17 @@ extern "C" int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_
     int rc = check_gemm_args(q_workspace, scale_workspace, packed, weight_scale, M, K, N, y,
                              y_dtype, nullptr);
     if (rc) return rc;
+    // one row (decode): both in one launch.  The same argument checks as the two calls make;
+    // past a few rounds of workgroups each would quantize again what one launch does once
+    if (M == 1 && x && scale_workspace && (!rms_input || rms_workspace) && precision_bits >= 2 &&
+        precision_bits <= 8 && valid_dtype(x_dtype) && K % 64 == 0 && K <= kQSmallMaxK &&
+        N <= kRowMaxN && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+        const float q_max = precision_bits <= 2 ? 1.0f : static_cast<float>((1 << (precision_bits - 1)) - 1);
+        const GemvProblem pb{packed, magnitude, bias, weight_scale, N, K};
+        launch_bitlinear_row(pb, x, x_dtype, q_max, rms_input != 0, y, y_dtype,
+                             static_cast<hipStream_t>(stream));
+        return check_launch("bitlinear_forward");
+    }
     rc = nsosx_quantize_act_i8(x, x_dtype, M, K, precision_bits, rms_input, q_workspace,
                                scale_workspace, rms_workspace, stream);
     if (rc) return rc;

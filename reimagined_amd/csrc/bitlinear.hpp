@@ -10,6 +10,7 @@
 #pragma once
 #include "common.hpp"
 #include "mamba2_step.hpp"
+#include "row_sum.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -53,97 +54,8 @@ __device__ __forceinline__ v4i unpack_word_mfma(uint32_t w) {
                (int)((w << 6) & 0xC0C0C0C0u)};
 }
 
-// ===========================================================================
-// Few rows with RMS_PERI (decode): the RMS pass and the quantization in one
-// launch.  A workgroup per row keeps the row in registers (8 elements per
-// thread and 2048-element chunk, K % 8 == 0, K <= 4096) and in LDS as floats;
-// lane 0 takes the in-order sum from LDS, the workgroup the absmax of x * inv
-// and the codes, with the operations of rms_inv_small_kernel and
-// quantize_rows_vec_kernel<DT, true> (so the same bits).
-// ===========================================================================
+// Longest row that a workgroup quantizes by itself (quantize_row_runs).
 constexpr int kQSmallMaxK = 4096;
-
-// One row by a 256-thread workgroup (K % 8 == 0, K <= 4096): with RMS, the squares
-// to s_row and the in-order sum by lane 0 (rms_inv_small_kernel's operations), then
-// the absmax of x * inv (x without RMS) and the codes, as quantize_rows_vec_kernel;
-// the codes to qrow and act_scale / inv (RMS) to *scale_out / *inv_out (global
-// memory or LDS).
-template <int DT, bool RMS>
-__device__ __forceinline__ void quantize_row_wg(const void* __restrict__ x, int64_t base, int K,
-                                                float q_max, float eps, float* s_row,
-                                                float* s_red, int8_t* qrow, float* scale_out,
-                                                float* inv_out) {
-    const int tid = threadIdx.x;
-    float v[2][8];
-    // the squares (each rounded on its own, as in the in-order sum) go to LDS, so the
-    // one lane that walks the row only adds: a chain of K dependent adds
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int e0 = (c * 256 + tid) * 8;
-        if (e0 < K) {
-            load8<DT>(x, base + e0, v[c]);
-            if (RMS) {
-                float q[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) q[j] = __fmul_rn(v[c][j], v[c][j]);
-                *reinterpret_cast<float4*>(s_row + e0) = make_float4(q[0], q[1], q[2], q[3]);
-                *reinterpret_cast<float4*>(s_row + e0 + 4) = make_float4(q[4], q[5], q[6], q[7]);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[c][j] = 0.0f;
-        }
-    }
-    if (RMS) {
-        __syncthreads();
-        if (tid == 0) {
-            float sum = 0.0f;
-#pragma unroll 8
-            for (int k = 0; k < K; k += 4) {
-                const float4 a = *reinterpret_cast<const float4*>(s_row + k);
-                sum = __fadd_rn(sum, a.x);
-                sum = __fadd_rn(sum, a.y);
-                sum = __fadd_rn(sum, a.z);
-                sum = __fadd_rn(sum, a.w);
-            }
-            const float mean = __fdiv_rn(sum, static_cast<float>(K));
-            const float inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, eps)));
-            s_red[4] = inv;
-            if (inv_out) *inv_out = inv;
-        }
-        __syncthreads();
-        const float inv = s_red[4];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[c][j] = __fmul_rn(v[c][j], inv);
-    }
-    float m = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(v[c][j]));
-    m = wave_max(m);
-    if ((tid & 63) == 0) s_red[tid >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-    const float denom = __fadd_rn(m, 1e-8f);
-    const float sc = __fdiv_rn(q_max, denom);
-    if (tid == 0) *scale_out = __fdiv_rn(denom, q_max);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int e0 = (c * 256 + tid) * 8;
-        if (e0 < K) {
-            float code[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) code[j] = clamp127(rintf(__fmul_rn(v[c][j], sc)));
-            uint2 out;
-            out.x = pack4_i8(code[0], code[1], code[2], code[3]);
-            out.y = pack4_i8(code[4], code[5], code[6], code[7]);
-            *reinterpret_cast<uint2*>(qrow + e0) = out;
-        }
-    }
-}
 
 // A group of a grouped GEMV with M >= 2 rows that the skinny MFMA body takes:
 // K = 1024 or 2048 (its fragments fit the launch's 64 KB of LDS) and whole
@@ -160,6 +72,9 @@ int launch_quantize_dt(const void* x, int dtype, int M, int K, int bits, int rms
 // gemv.hip: the VALU GEMV (M <= 8) on the reference words
 void launch_gemv(const GemvProblem& pb, const int8_t* q, const float* as, int M, void* y,
                  int y_dtype, int32_t* acc, hipStream_t st);
+// gemv.hip: quantization and GEMV of one row in one launch (K % 64 == 0, K <= kQSmallMaxK)
+void launch_bitlinear_row(const GemvProblem& pb, const void* x, int dtype, float q_max, bool rms,
+                          void* y, int y_dtype, hipStream_t st);
 // skinny.hip: the MFMA decode GEMV (2 <= M <= 32, skinny_ok), on the reference words
 // or (mfma_layout) the MFMA-layout words; and the grouped form for nsosx_grouped_gemv
 bool skinny_ok(int M, int K, int N);

@@ -5,7 +5,6 @@
 //   quantization  src/bitlinear.cpp:240-291, src/bitlinear_quantize_avx2.cpp:65-103
 //   RMS_PERI norm src/bitlinear.cpp:460-466, src/tensor.cpp:3455-3492
 #include "bitlinear.hpp"
-#include "row_sum.hpp"
 
 namespace nsosx {
 
@@ -290,13 +289,10 @@ __global__ __launch_bounds__(256) void rms_inv_small_kernel(const void* __restri
 //   int8 = clamp(code, -127, 127).
 // VEC: K % 8 == 0, every row 16-byte aligned -> 8 elements per lane-load,
 // the row kept in registers between the two passes when K <= 4096.
-// (load8 and the one-row quantize_row_wg live in bitlinear.hpp: the decode
-// projections of gemv.hip use them too.)
 // ===========================================================================
 // ===========================================================================
 // RMS_PERI + codes in one launch, a workgroup per row (row_sum.hpp takes the in-order sum;
 // by one lane walking the row from LDS it was 4.2 us of a call at K = 1024 and 16 us at 4096).
-// The absmax of x * inv is round(max|x| * inv): rounding is monotonic.
 // Time per call, us, before (a serial sum up to 1024 rows, two passes above) -> now:
 //   bf16   1 x 1024 6.4 -> 5.0    64 x 2048 11.4 -> 6.4    1024 x 4096 32.8 -> 11.6
 //   f32  300 x 768  6.8 -> 5.7  1500 x 2048 18.2 -> 9.6    3000 x 4096 38.8 -> 27.4
@@ -311,52 +307,11 @@ __global__ __launch_bounds__(512) void quantize_row_rms_kernel(const void* __res
                                                                int8_t* __restrict__ q,
                                                                float* __restrict__ act_scale) {
     extern __shared__ __align__(16) float s_dyn[];  // 8 floats per thread, then a SumRun each
-    __shared__ unsigned long long s_mask[8];
-    __shared__ float s_w[8], s_max[8], s_inv;
-    float* s_sq = s_dyn;
-    SumRun* s_run = reinterpret_cast<SumRun*>(s_dyn + 8 * blockDim.x);
+    __shared__ RowScratch scratch;
     const int64_t row = blockIdx.x;
-    const int tid = threadIdx.x;
-    const bool in = tid * 8 < K;  // K % 8 == 0
-    float v[8], sq[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = 0.0f;
-    if (in) load8<DT>(x, row * K + tid * 8, v);
-    float m = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        sq[j] = __fmul_rn(v[j], v[j]);
-        m = fmaxf(m, fabsf(v[j]));
-    }
-    *reinterpret_cast<float4*>(s_sq + tid * 8) = make_float4(sq[0], sq[1], sq[2], sq[3]);
-    *reinterpret_cast<float4*>(s_sq + tid * 8 + 4) = make_float4(sq[4], sq[5], sq[6], sq[7]);
-    m = wave_max(m);
-    if ((tid & 63) == 0) s_max[tid >> 6] = m;
-    // (adding the zeros past the row's end leaves the sum as it is)
-    const float sum = row_sum_in_order(sq, s_sq, s_run, s_w, s_mask);
-    if (tid == 0) {
-        const float mean = __fdiv_rn(sum, static_cast<float>(K));
-        const float inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, eps)));
-        s_inv = inv;
-        rms_inv[row] = inv;
-    }
-    __syncthreads();
-    const float inv = s_inv;
-    m = 0.0f;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = fmaxf(m, s_max[w]);
-    // an infinite x gives inf * 0, which the absmax of the products skips
-    m = fmaxf(0.0f, __fmul_rn(m, inv));
-    const float denom = __fadd_rn(m, 1e-8f);
-    const float sc = __fdiv_rn(q_max, denom);
-    if (tid == 0) act_scale[row] = __fdiv_rn(denom, q_max);
-    if (!in) return;
-    float code[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) code[j] = clamp127(rintf(__fmul_rn(__fmul_rn(v[j], inv), sc)));
-    uint2 out;
-    out.x = pack4_i8(code[0], code[1], code[2], code[3]);
-    out.y = pack4_i8(code[4], code[5], code[6], code[7]);
-    *reinterpret_cast<uint2*>(q + row * K + tid * 8) = out;
+    quantize_row_runs<DT, true, 8>(x, row * K, K, q_max, eps, s_dyn,
+                                   reinterpret_cast<SumRun*>(s_dyn + 8 * blockDim.x), scratch,
+                                   q + row * K, act_scale + row, rms_inv + row);
 }
 
 template <int DT, bool RMS>

@@ -10,7 +10,7 @@
 namespace nsosx {
 
 // ===========================================================================
-// Eight consecutive elements per thread.  The in-order float sum S <- round(S + v_k) is a chain
+// E (8 or 16) consecutive elements per thread.  The in-order float sum S <- round(S + v_k) is a chain
 // of K dependent adds (one lane walking the row from LDS: 8.8 cycles each, 4.2 us at
 // K = 1024, 16 us at 4096), but inside one binade of S its rounding depends on S only
 // through S's last bit: with S = 2^e + n ulp, round(S + v) - S is the same for every even n
@@ -21,7 +21,7 @@ namespace nsosx {
 //   1. every thread sums its squares; a scan gives each thread an estimate of S at its
 //      first element, hence the binade it expects, and the element (if any) at which S
 //      enters another one;
-//   2. each thread runs the two additions over its eight elements, before (A) and after (B)
+//   2. each thread runs the two additions over its elements, before (A) and after (B)
 //      that element; a segmented scan composes the increments of neighbouring threads;
 //   3. one wave walks the row's segments (about log2 K of them) with the true S in scalar
 //      registers: an increment per run, one real float add per crossing.  The estimate
@@ -67,16 +67,18 @@ __device__ __forceinline__ void sum_scan(int& d0, int& d1, int head) {
 
 __device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 
-// The in-order sum of the row's squares, in s_sq (thread t's: sq) with K = 8 * blockDim.x
-// entries, zeros past the row's end; returned to wave 0.  s_run: blockDim.x entries; s_w: 8
-// floats and 8 masks.
-__device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const float* s_sq,
+// The in-order sum of a row's squares (thread t's E: sq; all of them in s_sq, zeros past the
+// row's end) over the first `waves` waves of the workgroup; returned to wave 0, every thread
+// must call it.  s_run: an entry per thread; s_w, s_mask: one per wave.
+template <int E>
+__device__ __forceinline__ float row_sum_in_order(const float (&sq)[E], int waves, const float* s_sq,
                                                   SumRun* s_run, float* s_w,
                                                   unsigned long long* s_mask) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int waves = blockDim.x >> 6;
-    const float own = ((sq[0] + sq[1]) + (sq[2] + sq[3])) + ((sq[4] + sq[5]) + (sq[6] + sq[7]));
+    float own = 0.0f;
+#pragma unroll
+    for (int i = 0; i < E; i += 4) own += (sq[i] + sq[i + 1]) + (sq[i + 2] + sq[i + 3]);
     float incl = own;
     incl += __int_as_float(dpp0<kDppShr1>(__float_as_int(incl)));
     incl += __int_as_float(dpp0<kDppShr2>(__float_as_int(incl)));
@@ -99,14 +101,14 @@ __device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const fl
     uint32_t eb = ea;
     if (__ballot((__float_as_uint(r + own) & kExp) != ea) == 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < E; ++i) {
             t0 = __fadd_rn(t0, sq[i]);
             t1 = __fadd_rn(t1, sq[i]);
         }
     } else {
         float c0 = t0, c1 = t1;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < E; ++i) {
             r = __fadd_rn(r, sq[i]);
             const uint32_t en = __float_as_uint(r) & kExp;
             const bool cross = en != eb;
@@ -147,13 +149,17 @@ __device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const fl
     uint32_t s = 0;  // S's bits
     int pos = 0;     // elements added
     auto one_by_one = [&](int end) {  // at most to the end of pos's thread
-        const float4 a = *reinterpret_cast<const float4*>(s_sq + (pos & ~7));
-        const float4 b = *reinterpret_cast<const float4*>(s_sq + (pos & ~7) + 4);
-        const float c[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        const int lo = pos & 7, hi = end - (pos & ~7);
+        const int at = pos & ~(E - 1);
+        const int lo = pos - at, hi = end - at;
+        float c[E];
+#pragma unroll
+        for (int i = 0; i < E; i += 4) {
+            const float4 a = *reinterpret_cast<const float4*>(s_sq + at + i);
+            c[i] = a.x; c[i + 1] = a.y; c[i + 2] = a.z; c[i + 3] = a.w;
+        }
         float f = __uint_as_float(s);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < E; ++i) {
             const float n = __fadd_rn(f, c[i]);
             f = i >= lo && i < hi ? n : f;
         }
@@ -174,7 +180,7 @@ __device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const fl
                                                            : read_lane(cur.d0, to - 1));
             if ((s >> 23) == e && (whole >> 23) == e) {
                 s = whole;
-                pos = (first + to) * 8;
+                pos = (first + to) * E;
                 return;
             }
             int d0 = cur.d0, d1 = cur.d1;
@@ -186,14 +192,14 @@ __device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const fl
                     const int f = out ? __builtin_ctzll(out) : to;
                     if (f > from) {
                         s = (uint32_t)read_lane((int)n, f - 1);
-                        pos = (first + f) * 8;
+                        pos = (first + f) * E;
                     }
                     if (f == to) return;
                     from = f;
                 }
                 // S is not where it was expected (a crossing an element early or late): this
                 // thread's elements one by one, then the run from the next thread on
-                one_by_one((first + from + 1) * 8);
+                one_by_one((first + from + 1) * E);
                 if (++from == to) return;
                 if ((s >> 23) == e) {
                     d0 = cur.r0;
@@ -205,13 +211,13 @@ __device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const fl
         int from = 0;
         for (;;) {
             const int next = mask ? __builtin_ctzll(mask) : 64;
-            if (pos < (first + next) * 8) advance(from, next);
+            if (pos < (first + next) * E) advance(from, next);
             if (next == 64) break;
             mask &= mask - 1;
             const int meta = read_lane(cur.meta, next);
-            const int at_el = (first + next) * 8;
+            const int at_el = (first + next) * E;
             if (meta & kSumSerial) {
-                one_by_one(at_el + 8);
+                one_by_one(at_el + E);
                 from = next + 1;
             } else {
                 const int j = at_el + ((meta >> 16) & 15);
@@ -232,7 +238,83 @@ __device__ __forceinline__ float row_sum_in_order(const float (&sq)[8], const fl
     return __uint_as_float(s);
 }
 
-// LDS bytes of the row kernels: the squares and a SumRun per thread.
+// One row's int8 codes by a workgroup, E elements per thread (K <= E * blockDim.x, K % 8 == 0):
+// with RMS the in-order sum, then the absmax of x * inv (x without RMS) as round(max|x| * inv) --
+// rounding is monotonic -- and the codes with quantize_rows_vec_kernel's operations.  Codes to
+// qrow, act_scale / inv to *scale_out / *inv_out (global memory or LDS; inv_out may be null).
+// s_sq: E floats per thread, s_run: a SumRun per thread (both unused without RMS).
+struct RowScratch {
+    unsigned long long mask[8];
+    float w[8], max[8], inv;
+};
+
+template <int DT, bool RMS, int E>
+__device__ __forceinline__ void quantize_row_runs(const void* __restrict__ x, int64_t base, int K,
+                                                  float q_max, float eps, float* s_sq, SumRun* s_run,
+                                                  RowScratch& sc, int8_t* qrow, float* scale_out,
+                                                  float* inv_out) {
+    const int tid = threadIdx.x;
+    const int waves = blockDim.x >> 6;
+    float v[E];
+    float m = 0.0f;
+#pragma unroll
+    for (int c = 0; c < E; c += 8) {
+        float t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[j] = 0.0f;
+        if (tid * E + c < K) load8<DT>(x, base + tid * E + c, t);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[c + j] = t[j];
+            m = fmaxf(m, fabsf(t[j]));
+        }
+    }
+    m = wave_max(m);
+    if ((tid & 63) == 0) sc.max[tid >> 6] = m;
+    float inv = 1.0f;
+    if constexpr (RMS) {
+        float sq[E];
+#pragma unroll
+        for (int j = 0; j < E; ++j) sq[j] = __fmul_rn(v[j], v[j]);
+#pragma unroll
+        for (int j = 0; j < E; j += 4)
+            *reinterpret_cast<float4*>(s_sq + tid * E + j) = make_float4(sq[j], sq[j + 1], sq[j + 2], sq[j + 3]);
+        // (adding the zeros past the row's end leaves the sum as it is)
+        const float sum = row_sum_in_order<E>(sq, min(waves, (K + 64 * E - 1) / (64 * E)), s_sq, s_run,
+                                              sc.w, sc.mask);
+        if (tid == 0) {
+            const float mean = __fdiv_rn(sum, static_cast<float>(K));
+            const float one = __fdiv_rn(1.0f, sqrtf(__fadd_rn(mean, eps)));
+            sc.inv = one;
+            if (inv_out) *inv_out = one;
+        }
+    }
+    __syncthreads();
+    if (RMS) inv = sc.inv;
+    m = 0.0f;
+    for (int w = 0; w < waves; ++w) m = fmaxf(m, sc.max[w]);
+    // an infinite x gives inf * 0, which the absmax of the products skips
+    if (RMS) m = fmaxf(0.0f, __fmul_rn(m, inv));
+    const float denom = __fadd_rn(m, 1e-8f);
+    const float s = __fdiv_rn(q_max, denom);
+    if (tid == 0) *scale_out = __fdiv_rn(denom, q_max);
+#pragma unroll
+    for (int c = 0; c < E; c += 8) {
+        if (tid * E + c >= K) break;
+        float code[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float t = RMS ? __fmul_rn(v[c + j], inv) : v[c + j];
+            code[j] = clamp127(rintf(__fmul_rn(t, s)));
+        }
+        uint2 out;
+        out.x = pack4_i8(code[0], code[1], code[2], code[3]);
+        out.y = pack4_i8(code[4], code[5], code[6], code[7]);
+        *reinterpret_cast<uint2*>(qrow + tid * E + c) = out;
+    }
+}
+
+// LDS bytes of the one-row-per-workgroup kernels (E = 8): the squares and a SumRun per thread.
 inline unsigned row_sum_smem(int threads) {
     return threads * (8 * sizeof(float) + sizeof(SumRun));
 }

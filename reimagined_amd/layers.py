@@ -101,6 +101,11 @@ class BitLinear:
         m = x.shape[0]
         qw, sw, rw = self.workspace(m, x.device)
         st = _stream()
+        if m == 1 and marker is None:  # decode: quantization and GEMV in one launch
+            call("nsosx_bitlinear_forward", _p(x), ops._dt(x), _p(self.packed), self.weight_scale, m,
+                 self.in_features, self.out_features, self.bits, int(self.rms_input),
+                 _p(self.magnitude), _p(self.bias), _p(y), ops._dt(y), _p(qw), _p(sw), _p(rw), st)
+            return y
         call("nsosx_quantize_act_i8", _p(x), ops._dt(x), m, self.in_features, self.bits,
              int(self.rms_input), _p(qw), _p(sw), _p(rw), st)
         if marker:

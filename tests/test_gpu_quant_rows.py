@@ -65,3 +65,24 @@ def test_few_rows_equal_many_rows(dev, k):
     wq, ws = ops.quantize_activations_bitnet(many, 8, rms_input=True)
     np.testing.assert_array_equal(q.cpu().numpy(), wq[:64].cpu().numpy())
     np.testing.assert_array_equal(s.cpu().numpy(), ws[:64].cpu().numpy())
+
+
+@pytest.mark.parametrize("k,n", [(64, 48), (512, 33), (1024, 4096), (2048, 1000), (2112, 64),
+                                 (4096, 256)])
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("rms", [True, False])
+def test_one_row_forward_equals_quantize_then_gemv(dev, orc, k, n, bf16, rms):
+    """The one-launch forward of a row, bit for bit the oracle's quantization and affine."""
+    rng = np.random.default_rng(k + n)
+    packed, ws, codes = orc.pack_weights(rng.standard_normal((n, k)).astype(np.float32))
+    mag = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    pk = torch.from_numpy(packed.view(np.int32)).to(dev)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    for row in _rows(rng, k, bf16)[[0, 5, 7, 11, 12, 15]]:
+        x = torch.from_numpy(row[None]).to(torch.bfloat16 if bf16 else torch.float32).to(dev)
+        y = ops.bitnet_gemm_158bit_gpu(x, pk, ws, 1, k, n, magnitude=t(mag), bias=t(bias),
+                                       rms_input=rms)
+        want = orc.bitlinear_forward(row[None], packed, ws, n, rms_input=rms, magnitude=mag,
+                                     bias=bias)
+        np.testing.assert_array_equal(y.cpu().numpy(), want)
