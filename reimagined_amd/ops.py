@@ -26,11 +26,13 @@ def _dt(t: torch.Tensor) -> int:
 
 
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the current stream's handle without building a torch.cuda.Stream around it (1.5 us of
+    # host time per launch)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> torch.Tensor:
@@ -274,7 +276,7 @@ class LinearViewArray:
 
     @property
     def ptr(self):
-        return ctypes.c_void_p(self.tensor.data_ptr())
+        return self.tensor.data_ptr()
 
 
 class DecodeViewArray:
@@ -312,7 +314,7 @@ class DecodeViewArray:
 
     @property
     def ptr(self):
-        return ctypes.c_void_p(self.tensor.data_ptr())
+        return self.tensor.data_ptr()
 
 
 def grouped_decode_projections(views: DecodeViewArray, x: torch.Tensor, out_dtype=None,
