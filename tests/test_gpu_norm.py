@@ -71,6 +71,22 @@ def test_add_rmsnorm(dev, orc, dtype):
     np.testing.assert_array_equal(res2.float().cpu().numpy(), res.float().cpu().numpy())
 
 
+@pytest.mark.parametrize("dim", [1, 63, 64, 511, 513, 1025, 2047, 2048, 2049])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_add_rmsnorm_row_lengths(dev, orc, dim, dtype):
+    """Either side of the register forms' lengths (512, 1024, 2048) and ragged ones."""
+    rng = np.random.default_rng(dim)
+    x, d = (rng.standard_normal((5, dim)).astype(np.float32) for _ in range(2))
+    g = rng.uniform(0.5, 1.5, dim).astype(np.float32)
+    res, norm = ops.add_rmsnorm(_t(dev, x, dtype), _t(dev, d, dtype), _t(dev, g), eps=1e-6)
+    want = x + d if dtype == torch.float32 else _bf(_bf(x) + _bf(d))
+    np.testing.assert_array_equal(res.float().cpu().numpy(), want)
+    wn = orc.rmsnorm_gated(want, None, g, 1e-6)
+    # one bf16 rounding of the norm in bf16
+    tol = dict(rtol=1e-5, atol=1e-6) if dtype == torch.float32 else dict(rtol=2.0 ** -8, atol=1e-6)
+    np.testing.assert_allclose(norm.float().cpu().numpy(), wn, **tol)
+
+
 @pytest.mark.parametrize("width,bias,dtype", [(4, True, torch.float32), (1, False, torch.float32),
                                               (2, True, torch.float32), (4, True, torch.bfloat16)])
 def test_conv_step_chain_matches_oracle(dev, orc, width, bias, dtype):
