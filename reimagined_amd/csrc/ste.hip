@@ -11,7 +11,7 @@
 // GEMM for dmag (27 us) and a column reduction over two [M, N] arrays (145 us).  Now one
 // launch of 213 us for both contractions and the column sums (MFMA issue alone: 94 us at
 // the ~2.1 GHz it runs at; dW's strided gradient reads and its epilogue make its tiles the
-// longer ones), a forward and backward step 1061 -> 267 us.
+// longer ones), a forward and backward step 1061 -> 267 us (274 with the blocked sums).
 #include "row_sum.hpp"
 
 #include <cmath>
@@ -66,7 +66,7 @@ __device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& hi, ui
     lo = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), 0x07060302u);
 }
 
-// One 128 x 256 output tile: acc[rows][cols] = sum over the reduction of the gradient
+// One 128 x 256 output tile: total[rows][cols] = sum over the reduction of the gradient
 // operand (rows o0 .. of dW's j or d_act's m) and the exact operand bT (columns k0 ..).
 // DW: the gradient is read [reduction][output] (grad columns j, scaled by as[i]); else
 // [output][reduction] (grad rows m, scaled by mag[j]).  A thread cuts 8 reduction
@@ -77,7 +77,12 @@ __device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& hi, ui
 // colsum (DW): the thread's share of sum_i grad[i][j] for its column.
 template <bool DW, bool MAG>
 __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char* smem,
-                                         v16f (&acc)[2][2], float& colsum) {
+                                         v16f (&total)[2][2], float& colsum) {
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) acc[i][n] = total[i][n] = v16f{};
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int red = DW ? g.M : g.N;
@@ -261,6 +266,17 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
         for (; st + 1 < full; st += 2) {
             advance(st, s1);
             advance(st + 1, s0);
+            // the sums of 16 stages join the total: a chain of 96 MFMA additions, not one of
+            // 6 * full (4096 rows: error of dmag 6.2e-7 -> 2.5e-7 of its norm, float32 MFMA 3.0e-7)
+            if ((st & 14) == 14) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+                        total[i][n] += acc[i][n];
+                        acc[i][n] = v16f{};
+                    }
+            }
         }
         if (st < full) advance(st, s1);
         __syncthreads();  // (the stage past the end was read, though not used)
@@ -270,9 +286,13 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int n = 0; n < 2; ++n) acc[i][n] = v16f{};
+            for (int n = 0; n < 2; ++n) acc[i][n] = total[i][n] = v16f{};
         for (int st = 0; st * kTK < red; ++st) slow_stage(st, false);
     }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) total[i][n] += acc[i][n];
 }
 
 // dW and d_act tiles in one launch (each alone is 128 tiles at 4096 x 1024, together one
@@ -291,10 +311,6 @@ __global__ __launch_bounds__(kSteThreads, 2) void ste_gemm_kernel(SteArgs g) {
     const int wm = wave >> 2, wn = wave & 3;
     const int li = lane & 31, lh = lane >> 5;
     v16f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int n = 0; n < 2; ++n) acc[i][n] = v16f{};
     float colsum = 0.0f;
     const int k0 = (t < tiles_w ? t % tk : (t - tiles_w) % tk) * kTC;
 
