@@ -105,3 +105,47 @@ def test_ste_backward_matches_reference_golden(dev, orc, name):
     for key in ("dx", "dW", "dmag", "dbias"):
         if f"{name}__{key}" in g.files:
             _close(got[key], g[f"{name}__{key}"], rtol=1e-5, atol=1e-6, what=key)
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 4, 65), (63, 36, 66), (64, 64, 128), (65, 100, 129),
+                                   (130, 1000, 72), (257, 1024, 160), (10300, 260, 33)])
+@pytest.mark.parametrize("bf16,rms", [(False, False), (False, True), (True, False), (True, True)])
+def test_linear_f32_split_error_bound(dev, m, k, n, bf16, rms):
+    """The three-piece products at the edges of their 64 x 64 x 32 tiles, rows and weights over
+    twelve binades: within the rounding bound of a float sum of the row's products, K * 2^-24 of
+    the sum of their magnitudes (and a few roundings of the norm and the affine)."""
+    rng = np.random.default_rng(m + k + n)
+    x = (rng.standard_normal((m, k)) * 2.0 ** rng.uniform(-6, 6, (m, k))).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * 2.0 ** rng.uniform(-6, 6, (n, k))).astype(np.float32)
+    xt = torch.from_numpy(x).to(torch.bfloat16 if bf16 else torch.float32)
+    y = ops.linear_f32(xt.to(dev), torch.from_numpy(w).to(dev), rms).cpu().numpy()
+    xd = xt.double().numpy()
+    if rms:
+        xd = xd / np.sqrt((xd * xd).mean(1, keepdims=True) + 1e-6)
+    want, size = xd @ w.astype(np.float64).T, np.abs(xd) @ np.abs(w.astype(np.float64)).T
+    terms = k + 8 + (k if rms else 0)  # the RMS sum's own K roundings scale the row
+    assert np.all(np.abs(y - want) <= terms * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_linear_f32_split_keeps_infinities(dev, bf16):
+    """Infinities, NaN and values whose pieces would overflow give what the float dot product
+    gives: rows and columns that hold none are untouched."""
+    rng = np.random.default_rng(3)
+    m, k, n = 100, 96, 70
+    x, w = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (n, k)))
+    w = torch.from_numpy(w).to(torch.bfloat16).float().numpy()  # exact in one piece: m = l = 0
+    x[2, 3], x[5, 0], x[9, 95], x[40, 7] = np.inf, -np.inf, np.nan, 3.39e38
+    w[6, 9], w[11, 2], w[12] = np.inf, np.nan, 1e-3
+    xt = torch.from_numpy(x).to(torch.bfloat16 if bf16 else torch.float32)
+    y = ops.linear_f32(xt.to(dev), torch.from_numpy(w).to(dev)).cpu().numpy()
+    with np.errstate(invalid="ignore", over="ignore"):
+        # the 3.39e38 row times its weights stays in range in float64 and past it in float32
+        want = (xt.double().numpy()[:, None, :] * w.astype(np.float64)[None]).sum(-1).astype(np.float32)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(want))
+    np.testing.assert_array_equal(y[np.isinf(want)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    size = (np.abs(np.where(np.isfinite(x), x, 0)).astype(np.float64) @
+            np.abs(np.where(np.isfinite(w), w, 0)).astype(np.float64).T)
+    xs = xt.double().numpy()
+    assert np.all(np.abs(y[fine] - want[fine]) <= ((k + 8) * 2.0 ** -24 * (size + 2.0 ** -6 * np.abs(want)))[fine])
