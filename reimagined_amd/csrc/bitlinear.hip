@@ -117,14 +117,16 @@ extern "C" int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_
                              y_dtype, nullptr);
     if (rc) return rc;
     // one row (decode): both in one launch.  The same argument checks as the two calls make;
-    // past a few rounds of workgroups each would quantize again what one launch does once
+    // past a few rounds of workgroups each would quantize again what one launch does once, and
+    // an output written over its own input has to wait until every workgroup has read the row
     if (M == 1 && x && scale_workspace && (!rms_input || rms_workspace) && precision_bits >= 2 &&
         precision_bits <= 8 && valid_dtype(x_dtype) && K % 64 == 0 && K <= kQSmallMaxK &&
-        N <= kRowMaxN && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+        N <= kRowMaxN && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+        !overlaps(x, (int64_t)K * (x_dtype == NSOSX_F32 ? 4 : 2), y, (int64_t)N * (y_dtype == NSOSX_F32 ? 4 : 2))) {
         const float q_max = precision_bits <= 2 ? 1.0f : static_cast<float>((1 << (precision_bits - 1)) - 1);
         const GemvProblem pb{packed, magnitude, bias, weight_scale, N, K};
-        launch_bitlinear_row(pb, x, x_dtype, q_max, rms_input != 0, y, y_dtype,
-                             static_cast<hipStream_t>(stream));
+        launch_bitlinear_row(pb, x, x_dtype, q_max, rms_input != 0, q_workspace, scale_workspace,
+                             y, y_dtype, static_cast<hipStream_t>(stream));
         return check_launch("bitlinear_forward");
     }
     rc = nsosx_quantize_act_i8(x, x_dtype, M, K, precision_bits, rms_input, q_workspace,

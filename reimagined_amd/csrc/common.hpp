@@ -32,6 +32,12 @@ inline int check_launch(const char* what) {
 
 inline bool valid_dtype(int d) { return d == NSOSX_F32 || d == NSOSX_BF16; }
 
+// whether [a, a + a_bytes) and [b, b + b_bytes) share a byte
+inline bool overlaps(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + b_bytes && q < p + a_bytes;
+}
+
 // inv[m] = 1 / sqrt(mean_k x[m,k]^2 + eps), the row scale of Tensor::rmsnorm with its
 // in-order sum (bitlinear.hip); x [M, K] in `dtype`.
 void launch_rms_inv(const void* x, int dtype, int M, int K, float eps, float* inv,

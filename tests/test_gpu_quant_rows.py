@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from reimagined_amd import ops
+from reimagined_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +87,26 @@ def test_one_row_forward_equals_quantize_then_gemv(dev, orc, k, n, bf16, rms):
         want = orc.bitlinear_forward(row[None], packed, ws, n, rms_input=rms, magnitude=mag,
                                      bias=bias)
         np.testing.assert_array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("k,n", [(512, 512), (1024, 1000), (4096, 4096)])
+@pytest.mark.parametrize("rms", [True, False])
+def test_one_row_forward_keeps_the_codes_and_runs_in_place(dev, orc, k, n, rms):
+    """The workspaces hold the row's codes and scale afterwards, as a backward reads them, and y
+    may lie over x."""
+    rng = np.random.default_rng(k)
+    packed, ws, _ = orc.pack_weights(rng.standard_normal((n, k)).astype(np.float32))
+    pk = torch.from_numpy(packed.view(np.int32)).to(dev)
+    x = torch.randn((1, k), device=dev)
+    want_q, want_s = ops.quantize_activations_bitnet(x, 8, rms_input=rms)
+    want = ops.ternary_gemm(want_q, want_s, pk, ws, n)
+    q = torch.zeros((1, k), dtype=torch.int8, device=dev)
+    s, r = torch.zeros(1, device=dev), torch.zeros(1, device=dev)
+    buf = torch.zeros(max(k, n), device=dev)
+    for y in (torch.empty(n, device=dev), buf):
+        buf[:k] = x[0]
+        call("nsosx_bitlinear_forward", buf.data_ptr(), 0, pk.data_ptr(), ws, 1, k, n, 8, int(rms), None,
+             None, y.data_ptr(), 0, q.data_ptr(), s.data_ptr(), r.data_ptr(), None)
+        torch.cuda.synchronize()
+        assert torch.equal(q, want_q) and torch.equal(s, want_s)
+        assert torch.equal(y[:n], want.view(-1))
