@@ -1564,12 +1564,14 @@ extern "C" int nsosx_scan_fwd_planned(const void* x, int64_t x_stride, const flo
     const int Cn = resolve_chunk(num_seqs, total_tokens, H, P, N, chunk_tokens);
     // one A per head and a wide state: the scan as matrix products over chunks of 128 tokens,
     // where the recurrence would be chunked in time too (the gate and A forms it has no code
-    // for are)
+    // for are; nor does it run in place: a tile that is not finite reads its x again)
+    const int es = act_dtype == NSOSX_F32 ? 4 : 2;
     if (chunk_tokens < 0 && Cn > 0 && !a_per_state && !z &&
         ssd_shape(num_seqs, total_tokens, H, P, N) &&
-        (!conv_w || (conv_width >= 1 && conv_width <= 4)) && x && dt && A_log && B && C && D && y &&
+        (!conv_w || (conv_width >= 1 && conv_width <= 4)) && x_stride >= Dm && x && dt && A_log && B && C && D && y &&
         valid_dtype(act_dtype) && total_tokens > 0 &&
-        (reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16 == 0) {
+        (reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16 == 0 &&
+        !overlaps(x, ((int64_t)(total_tokens - 1) * x_stride + Dm) * es, y, (int64_t)total_tokens * Dm * es)) {
         const ScanWs ws = scan_ws_layout(workspace, num_seqs, total_tokens, Dm, N, kSsdChunk);
         hipStream_t st = static_cast<hipStream_t>(stream);
         hipLaunchKernelGGL(chunk_plan_kernel, dim3(1), dim3(1024), 0, st, cu_seqlens, num_seqs,

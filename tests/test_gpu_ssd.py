@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from reimagined_amd import ops
+from reimagined_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +103,24 @@ def test_matrix_scan_keeps_what_is_not_finite(dev, what):
         # (huge: sums of 1e38 terms that cancel, exact to the terms' size and not the sum's)
         atol = 1e-5 if what != "huge" else 1e-6 * b[ok].abs().max().item()
         torch.testing.assert_close(a[ok], b[ok], rtol=1e-4, atol=atol)
+
+
+def test_matrix_scan_refuses_and_runs_in_place_as_the_recurrence(dev):
+    """A row stride below H * P stays refused, and y over x gives what a buffer of its own does."""
+    lengths, H, N = [300, 129], 2, 64
+    d = _inputs(dev, lengths, H, N, 1, 4, torch.float32)
+    T, D = sum(lengths), H * 64
+    ws = torch.empty(int(ops.lib().nsosx_scan_fwd_workspace(2, T, H, 64, N, -1)), dtype=torch.uint8, device=dev)
+    p = lambda k: d[k].data_ptr()
+
+    def run(stride, y):
+        call("nsosx_scan_fwd_planned", p("x"), stride, None, None, 0, p("dt"), p("a_log"), 0, p("B"), p("C"),
+             p("D"), None, 0, p("cu"), 2, T, H, 64, N, 1, 0, None, None, y.data_ptr(), -1, ws.data_ptr(), None)
+        torch.cuda.synchronize()
+
+    y = torch.empty((T, D), device=dev)
+    with pytest.raises(Exception, match="stride"):
+        run(D - 64, y)
+    run(D, y)
+    run(D, d["x"])
+    torch.testing.assert_close(d["x"], y, rtol=1e-4, atol=1e-5)
