@@ -630,7 +630,7 @@ FP32_MFMA_PEAK_TFLOPS = 157.3
 
 
 def bench_linear_f32(torch, dev):
-    """BitLinear's float path (quantization-sensitive layers) on fp32 MFMA: the faithful
+    """BitLinear's float path (quantization-sensitive layers): the faithful
     Mamba-2 block's stacked B / C / dt projections over config 4's 40796 tokens (K 1024,
     N 2*16 + 32), and config 5's router gate (RMS_PERI, 8192 x 1024 -> 8).  Device time
     (graph replay): the gate's kernels run for less than the host's launch overhead."""
@@ -654,7 +654,8 @@ def bench_linear_f32(torch, dev):
 
 def bench_ste_backward(torch, dev):
     """The packed BitLinear STE backward at an in_proj-sized shape (M 4096 tokens, K 1024,
-    N 4096, RMS_PERI, magnitude): dW and d_act are 2*M*N*K fp32 MFMA flops each."""
+    N 4096, RMS_PERI, magnitude): dW and d_act are 2*M*N*K flops each (in bf16
+    pieces: the fraction of the fp32 MFMA peak can pass 1)."""
     from reimagined_amd import ops
     m, k, n = 4096, 1024, 4096
     rng = np.random.default_rng(9)

@@ -175,8 +175,8 @@ int nsosx_ternary_gemm_mfma(const int8_t* q, const float* act_scale, const uint3
 
 /* bitnet_gemm_158bit_gpu (include/bitnet_gpu_dispatch.h:46-51,
  * src/bitnet_gpu_dispatch.cpp:65-174): quantize x then ternary GEMM.
- * q_workspace: int8 [M, K]; scale_workspace: f32 [M];
- * rms_workspace: f32 [M] (only with rms_input). */
+ * q_workspace: int8 [M, K]; scale_workspace: f32 [M]: the codes and act_scale
+ * after the call; rms_workspace: f32 [M] (only with rms_input; scratch). */
 int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_t* packed,
                             float weight_scale, int M, int K, int N, int precision_bits,
                             int rms_input, const float* magnitude, const float* bias, void* y,
@@ -211,11 +211,13 @@ int nsosx_bitlinear_forward_noalloc(const void* x, int x_dtype, const uint32_t* 
  * f32 [N] or NULL; rms_workspace: f32 [M] when rms_input (required; the
  * skinny shapes below do not use it).  K % 4 == 0.
  * The dot products accumulate in fp32 in an order of their own: N <= 64 with
- * M > 16 on v_mfma_f32_16x16x4_f32 in one pass over x, the RMS sums of
- * squares taken on the way and 1 / rms applied to the dot products (equal to
- * the dot of the normalised row to rounding); other shapes with the
- * normalised input x * inv formed bit for bit as Tensor::rmsnorm, on
- * v_mfma_f32_32x32x2_f32 or, for N <= 16 or M <= 16, a wave reduction. */
+ * M > 16 (N <= 32 for M >= 10240 without rms_input) on v_mfma_f32_16x16x4_f32
+ * in one pass over x, the RMS sums of squares taken on the way and 1 / rms
+ * applied to the dot products (equal to the dot of the normalised row to
+ * rounding); other shapes with the normalised input x * inv formed bit for bit
+ * as Tensor::rmsnorm, on v_mfma_f32_32x32x16_bf16 with both operands cut into
+ * three bf16 pieces (float precision: the pieces' sum is the operand) or, for
+ * N <= 16 or M <= 16, a wave reduction. */
 int nsosx_linear_f32(const void* x, int x_dtype, int M, int K, const float* w, int N,
                      int rms_input, const float* magnitude, const float* bias, void* y,
                      int y_dtype, float* rms_workspace, void* stream);
@@ -371,7 +373,9 @@ int nsosx_conv_scan_fwd(const void* x_raw, int64_t x_stride, const float* conv_w
  *     differ by a few ulp);
  *   - chunk_tokens == 0: never chunk; -1: chunk when sequences x (H*P/16) <
  *     2048 and the sequences are at least two chunks long (chunk size aiming
- *     at 8192 waves, at least 64 tokens).
+ *     at 8192 waves, at least 64 tokens).  Where -1 chunks, one A per head of
+ *     P = 64 channels, N in {32, 48, 64}, no z and conv width <= 4 run as
+ *     matrix products over chunks of 128 tokens (float precision).
  * workspace: device, nsosx_scan_fwd_workspace(num_seqs, total_tokens, H, P,
  * N, chunk_tokens) bytes, 256-byte aligned.  Other arguments as above. */
 int64_t nsosx_scan_fwd_workspace(int num_seqs, int total_tokens, int H, int P, int N,

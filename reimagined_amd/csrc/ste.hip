@@ -9,9 +9,9 @@
 // sixteenth of the matrix-core time per pass.  Before: two fp32-MFMA GEMMs at the
 // card's fp32 rate (400 + 407 us at M = 4096, K = 1024, N = 4096), a full ternary
 // GEMM for dmag (27 us) and a column reduction over two [M, N] arrays (145 us).  Now one
-// launch of 213 us for both contractions and the column sums (MFMA issue alone: 94 us at
+// launch of about 220 us for both contractions and the column sums (MFMA issue alone: 94 us at
 // the ~2.1 GHz it runs at; dW's strided gradient reads and its epilogue make its tiles the
-// longer ones), a forward and backward step 1061 -> 267 us (274 with the blocked sums).
+// longer ones), a forward and backward step 1062 -> 273 us.
 #include "row_sum.hpp"
 
 #include <cmath>
