@@ -373,9 +373,7 @@ int nsosx_conv_scan_fwd(const void* x_raw, int64_t x_stride, const float* conv_w
  *     differ by a few ulp);
  *   - chunk_tokens == 0: never chunk; -1: chunk when sequences x (H*P/16) <
  *     2048 and the sequences are at least two chunks long (chunk size aiming
- *     at 8192 waves, at least 64 tokens).  Where -1 chunks, one A per head of
- *     P = 64 channels, N in {32, 48, 64}, no z and conv width <= 4 run as
- *     matrix products over chunks of 128 tokens (float precision).
+ *     at 8192 waves, at least 64 tokens).
  * workspace: device, nsosx_scan_fwd_workspace(num_seqs, total_tokens, H, P,
  * N, chunk_tokens) bytes, 256-byte aligned.  Other arguments as above. */
 int64_t nsosx_scan_fwd_workspace(int num_seqs, int total_tokens, int H, int P, int N,

@@ -12,7 +12,7 @@
 // exp2(delta * A2) with A2 = -exp(A_log) * log2(e) formed once per (channel,
 // state) in double and rounded to float; v_exp_f32 then costs one
 // transcendental per (token, channel, state).
-#include "scan_math.hpp"
+#include "common.hpp"
 #include "mamba2_step.hpp"
 
 #include <algorithm>
@@ -20,6 +20,44 @@
 #include <string>
 
 namespace nsosx {
+
+__device__ __forceinline__ float softplus_ref(float v) {
+    if (v > 20.0f) return v;
+    if (v < -20.0f) return expf(v);
+    return log1pf(expf(v));
+}
+
+__device__ __forceinline__ float a2_from_log(float a_log) {
+    return static_cast<float>(-exp(static_cast<double>(a_log)) * 1.4426950408889634);
+}
+
+__device__ __forceinline__ float dpp_xor1(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float dpp_xor2(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));
+}
+
+// Native-instruction forms of softplus and SiLU for the per-(token, channel)
+// terms (v_exp_f32 / v_log_f32 / v_rcp_f32, each about 1 ulp): log1p(e) is
+// taken as log(u) * e / (u - 1) with u = 1 + e, which cancels the rounding of
+// u (Kahan), so the relative error stays at a few ulp for all dt_raw.
+__device__ __forceinline__ float exp_native(float v) {
+    return __builtin_amdgcn_exp2f(v * 1.4426950408889634f);
+}
+
+__device__ __forceinline__ float softplus_fast(float v) {
+    if (v > 20.0f) return v;
+    if (v < -20.0f) return expf(v);
+    const float e = exp_native(v);
+    const float u = 1.0f + e;
+    if (u == 1.0f) return e;
+    return __builtin_amdgcn_logf(u) * 0.6931471805599453f * (e * __builtin_amdgcn_rcpf(u - 1.0f));
+}
+
+__device__ __forceinline__ float silu_fast(float v) {
+    return v * __builtin_amdgcn_rcpf(1.0f + exp_native(-v));
+}
 
 // ===========================================================================
 // Prefill scan.  A workgroup owns 64 channels of one sequence and walks its
@@ -349,6 +387,14 @@ __device__ __forceinline__ int quad_pick_sequence(const int32_t* cu, int num_seq
     return *s_pick;
 }
 
+
+// softplus_fast() without branches: the three regimes are formed and selected.
+__device__ __forceinline__ float softplus_sel(float v) {
+    const float e = exp_native(v);
+    const float u = 1.0f + e;
+    const float mid = __builtin_amdgcn_logf(u) * 0.6931471805599453f * (e * __builtin_amdgcn_rcpf(u - 1.0f));
+    return v > 20.0f ? v : (u == 1.0f ? e : mid);
+}
 
 // LOCAL: the first pass of the time-chunked scan: the recurrence only (no
 // readout, no output), writing each item's end state and sum of delta.
@@ -1443,39 +1489,6 @@ __global__ __launch_bounds__(256) void chunk_combine_kernel(
     }
 }
 
-// The carries of the matrix form, whose chunks all start from zero: before each chunk, and
-// after the last the sequence's final state.  Eight chunks' loads before the first store.
-__global__ __launch_bounds__(256) void ssd_combine_kernel(
-    const int32_t* __restrict__ first_chunk, int S, int D, int N, const float* __restrict__ a_log,
-    const float* __restrict__ local, const float* __restrict__ sum_dl,
-    const float* __restrict__ init_state, float* __restrict__ carry, float* __restrict__ final_state) {
-    const int per = D * N;  // chunks * D * N <= 2^28
-    const int s = blockIdx.y;
-    const int at = blockIdx.x * 256 + threadIdx.x;
-    if (at >= per) return;
-    const int c = at / N;
-    const float a2 = a2_from_log(a_log[c / 64]);
-    const int j0 = first_chunk[s], j1 = max(first_chunk[s + 1], j0);
-    float hs = init_state ? init_state[(int64_t)s * per + at] : 0.0f;
-    constexpr int U = 8;
-    for (int j = j0; j < j1; j += U) {
-        float lj[U], sum[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t r = min(j + u, j1 - 1);
-            lj[u] = local[r * per + at];
-            sum[u] = sum_dl[r * D + c];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (j + u >= j1) break;
-            carry[(int64_t)(j + u) * per + at] = hs;
-            hs = __fmaf_rn(__builtin_amdgcn_exp2f(a2 * sum[u]), hs, lj[u]);
-        }
-    }
-    if (final_state) final_state[(int64_t)s * per + at] = hs;
-}
-
 static int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
 // chunk_tokens < 0: chunk when sequences x 16-channel blocks give fewer than two
@@ -1537,11 +1550,7 @@ extern "C" int64_t nsosx_scan_fwd_workspace(int num_seqs, int total_tokens, int 
                                             int chunk_tokens) {
     if (num_seqs <= 0 || total_tokens < 0 || H <= 0 || P <= 0 || N <= 0) return 0;
     const int C = resolve_chunk(num_seqs, total_tokens, H, P, N, chunk_tokens);
-    int64_t bytes = scan_ws_layout(nullptr, num_seqs, total_tokens, H * P, N, C).bytes;
-    if (chunk_tokens < 0 && C > 0 && ssd_shape(num_seqs, total_tokens, H, P, N))  // the matrix form's chunks
-        bytes = std::max(bytes, scan_ws_layout(nullptr, num_seqs, total_tokens, H * P, N,
-                                               kSsdChunk).bytes);
-    return bytes;
+    return scan_ws_layout(nullptr, num_seqs, total_tokens, H * P, N, C).bytes;
 }
 
 extern "C" int nsosx_scan_fwd_planned(const void* x, int64_t x_stride, const float* conv_w,
@@ -1560,32 +1569,8 @@ extern "C" int nsosx_scan_fwd_planned(const void* x, int64_t x_stride, const flo
         return fail(NSOSX_ERR_INVALID, "scan_fwd_planned: bad shape (N <= 64, G > 0, H % G == 0)");
     if (chunk_tokens > 0 && chunk_tokens < 4)
         return fail(NSOSX_ERR_INVALID, "scan_fwd_planned: chunk_tokens must be >= 4, 0 or -1");
-    const int Dm = H * P;
     const int Cn = resolve_chunk(num_seqs, total_tokens, H, P, N, chunk_tokens);
-    // one A per head and a wide state: the scan as matrix products over chunks of 128 tokens,
-    // where the recurrence would be chunked in time too (the gate and A forms it has no code
-    // for are; nor does it run in place: a tile that is not finite reads its x again)
-    const int es = act_dtype == NSOSX_F32 ? 4 : 2;
-    if (chunk_tokens < 0 && Cn > 0 && !a_per_state && !z &&
-        ssd_shape(num_seqs, total_tokens, H, P, N) &&
-        (!conv_w || (conv_width >= 1 && conv_width <= 4)) && x_stride >= Dm && x && dt && A_log && B && C && D && y &&
-        valid_dtype(act_dtype) && total_tokens > 0 &&
-        (reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(C)) % 16 == 0 &&
-        !overlaps(x, ((int64_t)(total_tokens - 1) * x_stride + Dm) * es, y, (int64_t)total_tokens * Dm * es)) {
-        const ScanWs ws = scan_ws_layout(workspace, num_seqs, total_tokens, Dm, N, kSsdChunk);
-        hipStream_t st = static_cast<hipStream_t>(stream);
-        hipLaunchKernelGGL(chunk_plan_kernel, dim3(1), dim3(1024), 0, st, cu_seqlens, num_seqs,
-                           total_tokens, kSsdChunk, ws.maxc, ws.chunk_cu, ws.seq_start, ws.init_row,
-                           ws.state_row, ws.first_chunk);
-        const SsdArgs a{x, x_stride, conv_w, conv_b, conv_width, dt, A_log, B, C, D, ws.chunk_cu,
-                        ws.seq_start, ws.local, ws.sum_dl, ws.carry, y, total_tokens, H, N, G};
-        launch_ssd_states(a, act_dtype, ws.maxc, st);
-        hipLaunchKernelGGL(ssd_combine_kernel, dim3((Dm * N + 255) / 256, num_seqs), dim3(256), 0, st,
-                           ws.first_chunk, num_seqs, Dm, N, A_log, ws.local, ws.sum_dl,
-                           initial_state, ws.carry, final_state);
-        launch_ssd_output(a, act_dtype, ws.maxc, st);
-        return check_launch("scan_fwd_planned");
-    }
+    const int Dm = H * P;
     const ScanWs ws = scan_ws_layout(workspace, num_seqs, total_tokens, Dm, N, Cn);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (Cn == 0) {

@@ -1,5 +1,5 @@
-"""The matrix form of the scan (one A per head, d_state 32 .. 64) against the float64 recurrence, on
-both sides of its 128-token chunks and 32-token tiles, and against the sequential scan where the
+"""The scan at one A per head and d_state 32 .. 64 with the chunk length the library picks, against
+the float64 recurrence on both sides of chunk edges, and against the unchunked scan where the
 inputs are not finite.  Tolerance: the scan's own 1e-4 relative / 1e-5 absolute."""
 import numpy as np
 import pytest
@@ -56,7 +56,7 @@ def _float64(d, lengths, H, N, G, width, init):
 @pytest.mark.parametrize("lengths", [[129], [160, 127, 128, 129], [400, 0, 1], [97, 256], [31, 513, 32, 33]])
 @pytest.mark.parametrize("H,N,G,width,init", [(2, 64, 1, 4, False), (4, 48, 2, 4, True), (2, 32, 2, 0, True),
                                               (1, 64, 1, 2, True), (3, 32, 1, 1, False)])
-def test_matrix_scan_matches_float64(dev, lengths, H, N, G, width, init):
+def test_wide_scan_matches_float64(dev, lengths, H, N, G, width, init):
     d = _inputs(dev, lengths, H, N, G, sum(lengths) + N, torch.float32)
     y, fin = _run(d, H, N, G, width, init, -1)
     wy, wf = _float64(d, lengths, H, N, G, width, init)
@@ -65,7 +65,7 @@ def test_matrix_scan_matches_float64(dev, lengths, H, N, G, width, init):
 
 
 @pytest.mark.parametrize("dt_mean", [-8.0, -2.0, 3.0])
-def test_matrix_scan_no_less_exact_than_sequential(dev, dt_mean):
+def test_wide_scan_no_less_exact_than_sequential(dev, dt_mean):
     """Slow, ordinary and strong decays (a chunk's summed exponents reach -1e5)."""
     lengths, H, N, G = [700, 257, 64], 8, 64, 1
     d = _inputs(dev, lengths, H, N, G, 11, torch.float32, dt_mean)
@@ -76,7 +76,7 @@ def test_matrix_scan_no_less_exact_than_sequential(dev, dt_mean):
         assert err(a, w) <= max(1.2 * err(b, w), 2e-7), (dt_mean, err(a, w), err(b, w))
 
 
-def test_matrix_scan_bf16(dev):
+def test_wide_scan_bf16(dev):
     lengths, H, N, G = [230, 75], 4, 64, 1
     d = _inputs(dev, lengths, H, N, G, 5, torch.bfloat16)
     y, fin = _run(d, H, N, G, 4, True, -1)
@@ -86,7 +86,7 @@ def test_matrix_scan_bf16(dev):
 
 
 @pytest.mark.parametrize("what", ["x", "B", "C", "dt", "init", "huge"])
-def test_matrix_scan_keeps_what_is_not_finite(dev, what):
+def test_wide_scan_keeps_what_is_not_finite(dev, what):
     lengths, H, N, G = [200, 140], 2, 64, 1
     d = _inputs(dev, lengths, H, N, G, 8, torch.float32)
     if what == "init":
@@ -105,7 +105,7 @@ def test_matrix_scan_keeps_what_is_not_finite(dev, what):
         torch.testing.assert_close(a[ok], b[ok], rtol=1e-4, atol=atol)
 
 
-def test_matrix_scan_refuses_and_runs_in_place_as_the_recurrence(dev):
+def test_wide_scan_refuses_a_short_stride_and_runs_in_place(dev):
     """A row stride below H * P stays refused, and y over x gives what a buffer of its own does."""
     lengths, H, N = [300, 129], 2, 64
     d = _inputs(dev, lengths, H, N, 1, 4, torch.float32)
@@ -124,3 +124,16 @@ def test_matrix_scan_refuses_and_runs_in_place_as_the_recurrence(dev):
     run(D, y)
     run(D, d["x"])
     torch.testing.assert_close(d["x"], y, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("N,G,width,init,dtype", [(64, 1, 4, False, torch.float32), (64, 2, 0, True, torch.bfloat16),
+                                                  (48, 1, 2, True, torch.float32), (32, 1, 4, True, torch.float32)])
+@pytest.mark.parametrize("lengths", [[1025, 300], [2177], [129, 512]])
+def test_wide_scan_bits_are_the_recurrences(dev, lengths, N, G, width, init, dtype):
+    """The chunk length the library picks (here its least, 64 tokens) changes the carried states and
+    nothing else: the same bits as that length asked for.  A last-bit change of y moves int8 codes
+    of the projection behind the scan, which is 2e-4 of a block's output."""
+    H = 4
+    d = _inputs(dev, lengths, H, N, G, sum(lengths) + 3 * N, dtype)
+    for a, b in zip(_run(d, H, N, G, width, init, -1), _run(d, H, N, G, width, init, 64)):
+        assert torch.equal(a, b)
