@@ -211,13 +211,12 @@ int nsosx_bitlinear_forward_noalloc(const void* x, int x_dtype, const uint32_t* 
  * f32 [N] or NULL; rms_workspace: f32 [M] when rms_input (required; the
  * skinny shapes below do not use it).  K % 4 == 0.
  * The dot products accumulate in fp32 in an order of their own: N <= 64 with
- * M > 16 (N <= 32 for M >= 10240 without rms_input) on v_mfma_f32_16x16x4_f32
- * in one pass over x, the RMS sums of squares taken on the way and 1 / rms
- * applied to the dot products (equal to the dot of the normalised row to
- * rounding); other shapes with the normalised input x * inv formed bit for bit
- * as Tensor::rmsnorm, on v_mfma_f32_32x32x16_bf16 with both operands cut into
- * three bf16 pieces (float precision: the pieces' sum is the operand) or, for
- * N <= 16 or M <= 16, a wave reduction. */
+ * M > 16 on v_mfma_f32_16x16x4_f32 in one pass over x, the RMS sums of
+ * squares taken on the way and 1 / rms applied to the dot products (equal to
+ * the dot of the normalised row to rounding); other shapes with the
+ * normalised input x * inv formed bit for bit as Tensor::rmsnorm, on
+ * v_mfma_f32_32x32x2_f32 or, for N <= 16 or M <= 16, a wave reduction.
+ * y may lie over x (equal dtypes) where M > 16 and N = K <= 128, nowhere else. */
 int nsosx_linear_f32(const void* x, int x_dtype, int M, int K, const float* w, int N,
                      int rms_input, const float* magnitude, const float* bias, void* y,
                      int y_dtype, float* rms_workspace, void* stream);

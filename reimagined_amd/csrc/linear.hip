@@ -6,13 +6,21 @@
 //    faithful Mamba-2 block's B / C / dt projections and the MoE router's gate
 //    run this way (src/mamba2.cpp:588-599, 655-662; src/jamba.cpp:8086-8098).
 //
-// Two kernel families:
-//  * split_gemm_kernel: 64 x 64 outputs per workgroup on the bf16 matrix cores,
-//    both float32 operands cut into three bf16 pieces.
+// Three kernel families:
+//  * f32gemm_kernel (N > 64): a 128 x 128 output block per workgroup of four waves,
+//    each wave 64 x 64 as 2 x 2 tiles of v_mfma_f32_32x32x2_f32, 32-deep reduction
+//    stages double-buffered in LDS (one barrier per stage).  Both operands are
+//    staged reduction-major ([k][row] in LDS); the loader is a template on the
+//    dtype.  7078 x 1024 -> 160 (B / C / dt of the Mamba-2 block): 101 us on 112
+//    workgroups.  The same product on the bf16 matrix cores, operands in three
+//    pieces, took 33 us, but its sums come in another order: the block quantizes
+//    what follows, and the moved int8 codes were 2e-4 of its output.
+//  * skinny_f32_kernel (N <= 64, M > 16): one pass over x, K split over four waves.
 //  * dot_kernel: one wave per row of the large operand for the skinny shapes
-//    (router gates with N <= 16, decode with M <= 8), which leave an MFMA
+//    (router gates with N <= 16, decode with M <= 16), which leave an MFMA
 //    block mostly empty; the wave holds its row's K-chunks and dots them with
-//    the <= 16 rows of the small operand.
+//    the <= 16 rows of the small operand; dot_split_kernel the same with a
+//    workgroup per row.
 #include "common.hpp"
 
 #include <cmath>
@@ -20,224 +28,172 @@
 namespace nsosx {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
+constexpr int kGB = 128;        // output block (rows and columns)
+constexpr int kGK = 32;         // reduction depth of one LDS stage
+constexpr int kGLd = kGB + 4;   // LDS row pitch in floats (keeps 16-byte alignment)
 constexpr int kDotMax = 16;     // rows of the small operand in dot_kernel
 
-// ---------------------------------------------------------------------------
-// x @ W^T on the bf16 matrix cores.  Both operands are float32: each is cut into three bf16
-// pieces by rounding (8 significant bits each: x = h + m + l exactly), and of the nine
-// products the six down to 2^-18 of the whole are taken (h h; h m, m h; m m, h l, l h), each
-// exact in the MFMA's float32 sums; the rest is below 2^-26, a quarter of one float
-// rounding.  A bf16 x is its own first piece: three products.  Against float64 the error is
-// that of the float32 MFMA's sums or less (16 products are added per instruction, not 2).
-// A workgroup of four waves owns 64 x 64 outputs, a wave 32 x 32; 32-deep stages are cut on
-// the way into a double-buffered LDS ring (48 KB: three workgroups per CU, so that one cuts
-// while another multiplies -- both take about 400 cycles per wave and stage).
-// An output that is not finite is recomputed as a plain float32 dot product: the pieces of
-// an infinity or of a value near the top of the range are not numbers.
-// 7078 x 1024 -> 160 (B / C / dt of the Mamba-2 block): 101 us on v_mfma_f32_32x32x2_f32 with
-// 112 workgroups -> 33 us; 40796 x 1024 -> 64: 94 -> 50 us.
-// ---------------------------------------------------------------------------
-constexpr int kLB = 64;                     // output tile (rows and columns)
-constexpr int kLK = 32;                     // reduction depth of one LDS stage
-constexpr int kLPlane = kLB * kLK * 2;      // bytes of one bf16 piece of a stage
+// Operand layouts of f32gemm_kernel.  The output is [rows, cols] = [M, N]; the
+// reduction runs over K.  "o" below is the operand's output index (m for the
+// left operand, n for the right one), "k" the reduction index.
+enum OperandKind {
+    kRowK = 0,       // f32 [o][k] (row stride ld); optional per-o scale (RMS inverse)
+    kRowKBf16 = 1,   // bf16 [o][k]; optional per-o scale
+};
 
 struct GemmArgs {
-    const void* a;         // x [M, K], f32 or bf16
-    const float* a_scale;  // per row or null
-    const float* b;        // W [N, K]
+    const void* a;
+    int64_t lda;
+    const float* a_scale;
+    const void* b;
+    int64_t ldb;
+    const float* b_scale;
     int M, N, K;
     const float* mag;
     const float* bias;
     void* y;
+    int64_t ldy;
     int y_bf16;
 };
 
-// 16-byte chunk c (8 reduction elements) of tile row r, swizzled so that the 16 rows a
-// fragment read serves per clock cover all 64 banks.
-__device__ __forceinline__ int piece_at(int r, int c) { return r * 64 + ((c ^ ((r >> 2) & 3)) << 4); }
-
-__device__ __forceinline__ void split3_round(const float (&v)[8], u32x4 (&piece)[3]) {
+// Global -> registers: 16 floats per thread per stage, in the operand's own
+// order; st_tile() writes them reduction-major into the LDS stage.
+template <int KIND>
+__device__ __forceinline__ void ld_tile(const void* __restrict__ src, int64_t ld,
+                                        const float* __restrict__ scale, int o0, int k0, int O,
+                                        int Kr, float (&r)[16]) {
+    const int t = threadIdx.x;
+    {
+        const int kq = (t & 7) * 4;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        float a = v[2 * p], b = v[2 * p + 1];
+        for (int i = 0; i < 4; ++i) {
+            const int o = o0 + (t >> 3) + 32 * i;
+            const int k = k0 + kq;
+            float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (o < O && k < Kr) {
+                if constexpr (KIND == kRowK) {
+                    const float4 f = *reinterpret_cast<const float4*>(
+                        static_cast<const float*>(src) + (int64_t)o * ld + k);
+                    v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+                } else {
+                    const uint2 h = *reinterpret_cast<const uint2*>(
+                        static_cast<const uint16_t*>(src) + (int64_t)o * ld + k);
+                    v[0] = __uint_as_float(h.x << 16);
+                    v[1] = __uint_as_float(h.x & 0xffff0000u);
+                    v[2] = __uint_as_float(h.y << 16);
+                    v[3] = __uint_as_float(h.y & 0xffff0000u);
+                }
+                if (scale) {
+                    const float s = scale[o];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const uint32_t w = pack_bf16x2(a, b);
-            piece[i][p] = w;
-            a = __fsub_rn(a, __uint_as_float(w << 16));
-            b = __fsub_rn(b, __uint_as_float(w & 0xffff0000u));
+                    for (int c = 0; c < 4; ++c) v[c] = __fmul_rn(v[c], s);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) r[4 * i + c] = v[c];
         }
     }
 }
 
-template <int XDT, bool SCALED>
-__global__ __launch_bounds__(256, 3) void split_gemm_kernel(GemmArgs g, int ntn) {
-    constexpr int PA = XDT == NSOSX_BF16 && !SCALED ? 1 : 3;  // pieces of x
-    constexpr int kStage = (PA + 3) * kLPlane;
-    __shared__ __align__(16) char smem[2 * kStage];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // an XCD takes a run of consecutive tiles, columns fastest: they share x rows in its L2
-    const int per = gridDim.x / 8;
-    int t = blockIdx.x;
-    if (t < per * 8) t = (t % 8) * per + t / 8;
-    const int m0 = t / ntn * kLB, n0 = t % ntn * kLB;
-    const int full = g.K / kLK;
-    // this thread's chunk of both tiles: row tid / 4 (past the end: the last), chunk tid % 4
-    const int row = tid >> 2, chunk = tid & 3;
-    const int64_t arow = min(m0 + row, g.M - 1), brow = min(n0 + row, g.N - 1);
-    const float sc = SCALED ? g.a_scale[arow] : 1.0f;
-    const float* bsrc = g.b + brow * g.K;
-    struct Words {
-        float4 a[2], b[2];
-    };
-    auto load = [&](int st, Words& f) {
+template <int KIND>
+__device__ __forceinline__ void st_tile(float* __restrict__ s, const float (&r)[16]) {
+    const int t = threadIdx.x;
+    {
+        const int kq = (t & 7) * 4;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            // (past the end, and a stage cut by K: the last words again; K % 4 == 0)
-            const int at = min(st * kLK + chunk * 8 + 4 * h, g.K - 4);
-            float4 (&fa)[2] = f.a, (&fb)[2] = f.b;
-            if constexpr (XDT == NSOSX_F32) {
-                fa[h] = *reinterpret_cast<const float4*>(static_cast<const float*>(g.a) + arow * g.K + at);
-            } else {
-                const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(g.a) +
-                                                               arow * g.K + at);
-                fa[h] = make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u),
-                                    __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u));
-            }
-            fb[h] = *reinterpret_cast<const float4*>(bsrc + at);
+        for (int i = 0; i < 4; ++i) {
+            const int o = (t >> 3) + 32 * i;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[(kq + c) * kGLd + o] = r[4 * i + c];
         }
-    };
-    const int at = piece_at(row, chunk);
-    auto store = [&](int st, const Words& f, bool cut) {
-        char* s = smem + (st & 1) * kStage;
-        float a[8] = {f.a[0].x, f.a[0].y, f.a[0].z, f.a[0].w, f.a[1].x, f.a[1].y, f.a[1].z, f.a[1].w};
-        float b[8] = {f.b[0].x, f.b[0].y, f.b[0].z, f.b[0].w, f.b[1].x, f.b[1].y, f.b[1].z, f.b[1].w};
-        if (cut) {  // zeros past K
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (full * kLK + chunk * 8 + e >= g.K) a[e] = b[e] = 0.0f;
-        }
-        if (SCALED)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) a[e] = __fmul_rn(a[e], sc);
-        u32x4 piece[3];
-        split3_round(a, piece);
-#pragma unroll
-        for (int p = 0; p < PA; ++p) *reinterpret_cast<u32x4*>(s + p * kLPlane + at) = piece[p];
-        split3_round(b, piece);
-#pragma unroll
-        for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(s + (PA + p) * kLPlane + at) = piece[p];
-    };
-    v16f acc = {}, low = {};
+    }
+}
+
+template <int AK, int BK>
+__global__ __launch_bounds__(256, 2) void f32gemm_kernel(GemmArgs g) {
+    __shared__ __align__(16) float sA[2][kGK * kGLd];
+    __shared__ __align__(16) float sB[2][kGK * kGLd];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    const int li = lane & 31, lh = lane >> 5;
-    auto contract = [&](int st) {
-        const char* s = smem + (st & 1) * kStage;
+    const int m0 = blockIdx.x * kGB, n0 = blockIdx.y * kGB;
+    const int stages = (g.K + kGK - 1) / kGK;
+
+    v16f acc[2][2];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            v8bf a[PA], b[3];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int p = 0; p < PA; ++p)
-                a[p] = *reinterpret_cast<const v8bf*>(s + p * kLPlane + piece_at(wm * 32 + li, 2 * ks + lh));
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-                b[p] = *reinterpret_cast<const v8bf*>(s + (PA + p) * kLPlane +
-                                                      piece_at(wn * 32 + li, 2 * ks + lh));
-#pragma unroll
-            for (int d = 2; d >= 1; --d)
-#pragma unroll
-                for (int p = 0; p < PA; ++p)
-                    if (d - p >= 0)
-                        low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p], b[d - p], low, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    float ra[16], rb[16];
+    ld_tile<AK>(g.a, g.lda, g.a_scale, m0, 0, g.M, g.K, ra);
+    ld_tile<BK>(g.b, g.ldb, g.b_scale, n0, 0, g.N, g.K, rb);
+    st_tile<AK>(sA[0], ra);
+    st_tile<BK>(sB[0], rb);
+    __syncthreads();
+
+    const int fr = lane >> 5;   // reduction row of this lane's fragment element
+    const int fc = lane & 31;   // output index within a 32-wide tile
+    for (int st = 0; st < stages; ++st) {
+        const int cur = st & 1;
+        const bool more = st + 1 < stages;
+        if (more) {
+            ld_tile<AK>(g.a, g.lda, g.a_scale, m0, (st + 1) * kGK, g.M, g.K, ra);
+            ld_tile<BK>(g.b, g.ldb, g.b_scale, n0, (st + 1) * kGK, g.N, g.K, rb);
         }
-    };
-    // one stage's instructions in order: its fragment reads, then each MFMA with a share of the
-    // next stage's cut in its shadow (a stage's chain of 12 MFMAs and 110 VALU one after the
-    // other leaves a CU with one workgroup half idle)
-    auto order = [&]() {
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * (PA + 3), 0);  // LDS reads
+        const float* a = sA[cur] + wm * 64 + fc;
+        const float* b = sB[cur] + wn * 64 + fc;
 #pragma unroll
-        for (int i = 0; i < 2 * (PA == 1 ? 3 : 6); ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);  // VALU
+        for (int kk = 0; kk < kGK; kk += 2) {
+            const int off = (kk + fr) * kGLd;
+            const float a0 = a[off], a1 = a[off + 32];
+            const float b0 = b[off], b1 = b[off + 32];
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // stage st in LDS, st + 1 and st + 2 in flight in f1 / f0 (loads past the end re-read the last
-    // words; what they leave in the ring is not contracted)
-    Words f0, f1;
-    if (full > 0) {
-        load(0, f0);
-        __builtin_amdgcn_sched_barrier(0);
-        load(1, f1);
-        __builtin_amdgcn_sched_barrier(0);
-        store(0, f0, false);
-        __builtin_amdgcn_sched_barrier(0);
-        load(2, f0);
-        __syncthreads();
-        int st = 0;
-        for (; st + 1 < full; st += 2) {
-            contract(st);
-            store(st + 1, f1, false);
-            load(st + 3, f1);
-            order();
-            __syncthreads();
-            contract(st + 1);
-            store(st + 2, f0, false);
-            load(st + 4, f0);
-            order();
-            __syncthreads();
+        if (more) {
+            // the other buffer was last read before the previous stage's barrier
+            st_tile<AK>(sA[cur ^ 1], ra);
+            st_tile<BK>(sB[cur ^ 1], rb);
         }
-        if (st < full) contract(st);
         __syncthreads();
-    }
-    if (full * kLK < g.K) {  // the last stage, cut by K
-        load(full, f0);
-        store(0, f0, true);
-        __syncthreads();
-        contract(0);
     }
 
-    // D layout of the 32x32 MFMA: register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4,
-    // column l % 32
-    const int n = n0 + wn * 32 + li;
-    if (n >= g.N) return;
-    const float mg = g.mag ? g.mag[n] : 1.0f;
-    const float bs = g.bias ? g.bias[n] : 0.0f;
+    // C tile layout of the 32x32 MFMA: register r of lane l holds
+    // row 8*(r/4) + 4*(l/32) + r%4, column l%32.
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-        if (m >= g.M) continue;
-        float v = acc[r] + low[r];
-        if (!(fabsf(v) < __builtin_inff())) {
-            v = 0.0f;
-            for (int k = 0; k < g.K; ++k) {
-                float xv = load_act<XDT>(g.a, (int64_t)m * g.K + k);
-                if (SCALED) xv = __fmul_rn(xv, g.a_scale[m]);
-                v = __fmaf_rn(xv, g.b[(int64_t)n * g.K + k], v);
+    for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < 2; ++ni) {
+            const int n = n0 + wn * 64 + ni * 32 + fc;
+            if (n >= g.N) continue;
+            float mg = 1.0f, bs = 0.0f;
+            if (g.mag) mg = g.mag[n];
+            if (g.bias) bs = g.bias[n];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + wm * 64 + mi * 32 + 8 * (r >> 2) + 4 * fr + (r & 3);
+                if (m >= g.M) continue;
+                float v = acc[mi][ni][r];
+                if (g.mag) v = __fmul_rn(v, mg);
+                if (g.bias) v = __fadd_rn(v, bs);
+                if (g.y_bf16)
+                    static_cast<uint16_t*>(g.y)[(int64_t)m * g.ldy + n] = f32_to_bf16(v);
+                else
+                    static_cast<float*>(g.y)[(int64_t)m * g.ldy + n] = v;
             }
         }
-        if (g.mag) v = __fmul_rn(v, mg);
-        if (g.bias) v = __fadd_rn(v, bs);
-        if (g.y_bf16) static_cast<uint16_t*>(g.y)[(int64_t)m * g.N + n] = f32_to_bf16(v);
-        else static_cast<float*>(g.y)[(int64_t)m * g.N + n] = v;
-    }
 }
 
-static void launch_split_gemm(const GemmArgs& g, int x_dtype, hipStream_t st) {
-    const int ntn = (g.N + kLB - 1) / kLB;
-    const dim3 grid((unsigned)(((int64_t)g.M + kLB - 1) / kLB * ntn)), block(256);
-    if (x_dtype == NSOSX_F32) {
-        if (g.a_scale) hipLaunchKernelGGL((split_gemm_kernel<NSOSX_F32, true>), grid, block, 0, st, g, ntn);
-        else hipLaunchKernelGGL((split_gemm_kernel<NSOSX_F32, false>), grid, block, 0, st, g, ntn);
-    } else {
-        if (g.a_scale) hipLaunchKernelGGL((split_gemm_kernel<NSOSX_BF16, true>), grid, block, 0, st, g, ntn);
-        else hipLaunchKernelGGL((split_gemm_kernel<NSOSX_BF16, false>), grid, block, 0, st, g, ntn);
-    }
+template <int AK, int BK>
+static void launch_f32gemm(const GemmArgs& g, hipStream_t st) {
+    const dim3 grid((g.M + kGB - 1) / kGB, (g.N + kGB - 1) / kGB);
+    hipLaunchKernelGGL((f32gemm_kernel<AK, BK>), grid, dim3(256), 0, st, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -604,9 +560,7 @@ extern "C" int nsosx_linear_f32(const void* x, int x_dtype, int M, int K, const 
     // on the way and the 1 / rms applied to the row's dot products (equal to the dot of
     // the normalised row to rounding; bf16 rows are read 16 bytes at a time: K % 8 keeps
     // them aligned)
-    // (33 .. 64 columns of many rows without RMS_PERI go to the split GEMM: 94 -> 50 us at
-    // 40796 x 1024 -> 64; at 7078 rows its 111 workgroups take 26 us against 20)
-    if (N <= (rms_input || M < 10240 ? kSkinnyMaxN : 32) && M > kDotMax && (x_dtype == NSOSX_F32 || K % 8 == 0)) {
+    if (N <= kSkinnyMaxN && M > kDotMax && (x_dtype == NSOSX_F32 || K % 8 == 0)) {
         if (x_dtype == NSOSX_F32)
             launch_skinny<NSOSX_F32>(x, rms_input, w, M, N, K, magnitude, bias, y, ybf, st);
         else
@@ -640,7 +594,12 @@ extern "C" int nsosx_linear_f32(const void* x, int x_dtype, int M, int K, const 
 #undef NSOSX_DOT
         return check_launch("linear_f32");
     }
-    const GemmArgs g{x, inv, w, M, N, K, magnitude, bias, y, ybf};
-    launch_split_gemm(g, x_dtype, st);
+    GemmArgs g{};
+    g.a = x; g.lda = K; g.a_scale = inv;
+    g.b = w; g.ldb = K; g.b_scale = nullptr;
+    g.M = M; g.N = N; g.K = K;
+    g.mag = magnitude; g.bias = bias; g.y = y; g.ldy = N; g.y_bf16 = ybf;
+    if (x_dtype == NSOSX_F32) launch_f32gemm<kRowK, kRowK>(g, st);
+    else launch_f32gemm<kRowKBf16, kRowK>(g, st);
     return check_launch("linear_f32");
 }

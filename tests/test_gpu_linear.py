@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from reimagined_amd import ops
+from reimagined_amd._lib import call
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden", "bitlinear_ref.npz")
@@ -110,9 +111,9 @@ def test_ste_backward_matches_reference_golden(dev, orc, name):
 @pytest.mark.parametrize("m,k,n", [(17, 4, 65), (63, 36, 66), (64, 64, 128), (65, 100, 129),
                                    (130, 1000, 72), (257, 1024, 160), (10300, 260, 33)])
 @pytest.mark.parametrize("bf16,rms", [(False, False), (False, True), (True, False), (True, True)])
-def test_linear_f32_split_error_bound(dev, m, k, n, bf16, rms):
-    """The three-piece products at the edges of their 64 x 64 x 32 tiles, rows and weights over
-    twelve binades: within the rounding bound of a float sum of the row's products, K * 2^-24 of
+def test_linear_f32_error_bound(dev, m, k, n, bf16, rms):
+    """The matrix products around their tiles' edges, rows and weights over twelve binades:
+    within the rounding bound of a float sum of the row's products, K * 2^-24 of
     the sum of their magnitudes (and a few roundings of the norm and the affine)."""
     rng = np.random.default_rng(m + k + n)
     x = (rng.standard_normal((m, k)) * 2.0 ** rng.uniform(-6, 6, (m, k))).astype(np.float32)
@@ -128,13 +129,13 @@ def test_linear_f32_split_error_bound(dev, m, k, n, bf16, rms):
 
 
 @pytest.mark.parametrize("bf16", [True, False])
-def test_linear_f32_split_keeps_infinities(dev, bf16):
-    """Infinities, NaN and values whose pieces would overflow give what the float dot product
+def test_linear_f32_keeps_infinities(dev, bf16):
+    """Infinities, NaN and values near the top of the range give what the float dot product
     gives: rows and columns that hold none are untouched."""
     rng = np.random.default_rng(3)
     m, k, n = 100, 96, 70
     x, w = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (n, k)))
-    w = torch.from_numpy(w).to(torch.bfloat16).float().numpy()  # exact in one piece: m = l = 0
+    w = torch.from_numpy(w).to(torch.bfloat16).float().numpy()
     x[2, 3], x[5, 0], x[9, 95], x[40, 7] = np.inf, -np.inf, np.nan, 3.39e38
     w[6, 9], w[11, 2], w[12] = np.inf, np.nan, 1e-3
     xt = torch.from_numpy(x).to(torch.bfloat16 if bf16 else torch.float32)
@@ -149,3 +150,17 @@ def test_linear_f32_split_keeps_infinities(dev, bf16):
             np.abs(np.where(np.isfinite(w), w, 0)).astype(np.float64).T)
     xs = xt.double().numpy()
     assert np.all(np.abs(y[fine] - want[fine]) <= ((k + 8) * 2.0 ** -24 * (size + 2.0 ** -6 * np.abs(want)))[fine])
+
+
+@pytest.mark.parametrize("m,n", [(17, 64), (300, 100), (129, 128)])
+@pytest.mark.parametrize("rms", [False, True])
+def test_linear_f32_in_place(dev, m, n, rms):
+    """y over x where a workgroup owns whole rows (M > 16, N = K <= 128): the same bits as y apart."""
+    rng = np.random.default_rng(m + n)
+    x, w = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).to(dev) for s in ((m, n), (n, n)))
+    want = ops.linear_f32(x, w, rms)
+    ws = torch.empty(m, device=dev)
+    call("nsosx_linear_f32", x.data_ptr(), 0, m, n, w.data_ptr(), n, int(rms), None, None, x.data_ptr(), 0,
+         ws.data_ptr(), None)
+    torch.cuda.synchronize()
+    assert torch.equal(x, want)
