@@ -19,8 +19,7 @@
 //  * dot_kernel: one wave per row of the large operand for the skinny shapes
 //    (router gates with N <= 16, decode with M <= 16), which leave an MFMA
 //    block mostly empty; the wave holds its row's K-chunks and dots them with
-//    the <= 16 rows of the small operand; dot_split_kernel the same with a
-//    workgroup per row.
+//    the small operand's rows, four of them or all <= 16.
 #include "common.hpp"
 
 #include <cmath>
@@ -201,6 +200,8 @@ static void launch_f32gemm(const GemmArgs& g, hipStream_t st) {
 //   PER_M: wave m holds x[m] (times inv[m]) and dots it with the N <= 16 rows
 //          of W (router gates);
 //   else : wave n holds W[n] and dots it with the M <= 16 rows of x (decode).
+// A workgroup row (blockIdx.y) takes JM of the small rows.  A pair's sum is one lane chain over
+// K and a tree across the lanes whatever JM is, so the split changes no bit.
 // ---------------------------------------------------------------------------
 template <int XDT, bool PER_M, int JM>
 __global__ __launch_bounds__(256) void dot_kernel(const void* __restrict__ x,
@@ -213,6 +214,7 @@ __global__ __launch_bounds__(256) void dot_kernel(const void* __restrict__ x,
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int nbig = PER_M ? M : N;
     const int nsmall = PER_M ? N : M;
+    const int j0 = blockIdx.y * JM;  // this workgroup's first small row
     if (row >= nbig) return;
     float acc[JM];
 #pragma unroll
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(256) void dot_kernel(const void* __restrict__ x,
             else load4(w, NSOSX_F32, (int64_t)row * K + k, mine[u]);
 #pragma unroll
             for (int j = 0; j < JM; ++j) {
-                const int jj = min(j, nsmall - 1);
+                const int jj = min(j0 + j, nsmall - 1);
                 if (PER_M) load4(w, NSOSX_F32, (int64_t)jj * K + k, other[u][j]);
                 else xval4(jj, k, other[u][j]);
             }
@@ -259,98 +261,26 @@ __global__ __launch_bounds__(256) void dot_kernel(const void* __restrict__ x,
             if (k0 + 256 * u >= K) break;
 #pragma unroll
             for (int j = 0; j < JM; ++j)
-                if (j < nsmall)
+                if (j0 + j < nsmall)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[j] = __fmaf_rn(mine[u][e], other[u][j][e], acc[j]);
         }
     }
 #pragma unroll
     for (int j = 0; j < JM; ++j) {
-        if (j >= nsmall) continue;
+        if (j0 + j >= nsmall) continue;
         float v = acc[j];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) v = __fadd_rn(v, __shfl_xor(v, off));
         if (lane == 0) {
-            const int m = PER_M ? row : j;
-            const int n = PER_M ? j : row;
+            const int m = PER_M ? row : j0 + j;
+            const int n = PER_M ? j0 + j : row;
             if (mag) v = __fmul_rn(v, mag[n]);
             if (bias) v = __fadd_rn(v, bias[n]);
             if (y_bf16) static_cast<uint16_t*>(y)[(int64_t)m * N + n] = f32_to_bf16(v);
             else static_cast<float*>(y)[(int64_t)m * N + n] = v;
         }
     }
-}
-
-// 5 .. 16 small rows and too few big ones to fill the chip with a wave each (B / C / dt of a
-// decode batch: 160 rows of W, 40 workgroups): a workgroup per big row, its waves 256 elements of
-// K apart, the 16 partial sums of its 256 lanes added through LDS in a fixed order.  16 x 1024 ->
-// 160: 10.6 -> 3.7 us.
-template <int XDT, bool PER_M>
-__global__ __launch_bounds__(256) void dot_split_kernel(const void* __restrict__ x,
-                                                        const float* __restrict__ inv,
-                                                        const float* __restrict__ w, int M, int N,
-                                                        int K, const float* __restrict__ mag,
-                                                        const float* __restrict__ bias, void* y,
-                                                        int y_bf16) {
-    __shared__ float s_part[kDotMax][256 + 16];
-    const int tid = threadIdx.x;
-    const int row = blockIdx.x;
-    const int nsmall = PER_M ? N : M;
-    auto load4 = [&](const void* base, int dt, int64_t off, float v[4]) {
-        if (dt == NSOSX_F32) {
-            const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + off);
-            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        } else {
-            const uint2 a = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + off);
-            v[0] = __uint_as_float(a.x << 16); v[1] = __uint_as_float(a.x & 0xFFFF0000u);
-            v[2] = __uint_as_float(a.y << 16); v[3] = __uint_as_float(a.y & 0xFFFF0000u);
-        }
-    };
-    float acc[kDotMax];
-#pragma unroll
-    for (int j = 0; j < kDotMax; ++j) acc[j] = 0.0f;
-    for (int k = 4 * tid; k < K; k += 1024) {  // K % 4 == 0
-        float mine[4], other[kDotMax][4];
-        load4(PER_M ? x : static_cast<const void*>(w), PER_M ? XDT : NSOSX_F32, (int64_t)row * K + k, mine);
-#pragma unroll
-        for (int j = 0; j < kDotMax; ++j)  // rows past nsmall re-read the last, not stored
-            load4(PER_M ? static_cast<const void*>(w) : x, PER_M ? NSOSX_F32 : XDT,
-                  (int64_t)min(j, nsmall - 1) * K + k, other[j]);
-        if (inv) {
-#pragma unroll
-            for (int j = 0; j < (PER_M ? 1 : kDotMax); ++j) {
-                const float s = inv[PER_M ? row : min(j, nsmall - 1)];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (PER_M) mine[e] = __fmul_rn(mine[e], s);
-                    else other[j][e] = __fmul_rn(other[j][e], s);
-                }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kDotMax; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[j] = __fmaf_rn(mine[e], other[j][e], acc[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < kDotMax; ++j) s_part[j][tid + (tid >> 4)] = acc[j];
-    __syncthreads();
-    // thread (j, p): lanes 16 p .. 16 p + 15 of sum j, then across p
-    const int j = tid >> 4, p = tid & 15;
-    float v = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v = __fadd_rn(v, s_part[j][17 * p + i]);
-    v = __fadd_rn(v, lane_xor<8>(v));
-    v = __fadd_rn(v, lane_xor<4>(v));
-    v = __fadd_rn(v, lane_xor<2>(v));
-    v = __fadd_rn(v, lane_xor<1>(v));
-    if (p != 0 || j >= nsmall) return;
-    const int m = PER_M ? row : j;
-    const int n = PER_M ? j : row;
-    if (mag) v = __fmul_rn(v, mag[n]);
-    if (bias) v = __fadd_rn(v, bias[n]);
-    if (y_bf16) static_cast<uint16_t*>(y)[(int64_t)m * N + n] = f32_to_bf16(v);
-    else static_cast<float*>(y)[(int64_t)m * N + n] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -572,18 +502,19 @@ extern "C" int nsosx_linear_f32(const void* x, int x_dtype, int M, int K, const 
     if (N <= kDotMax || M <= kDotMax) {
         const bool per_m = N <= kDotMax && !(M <= kDotMax && M < N);
         const int rows = per_m ? M : N;
-        const dim3 grid((rows + 3) / 4);
         const int nsmall = per_m ? N : M;
+        // 5 .. 16 small rows of up to 2048 big ones: four small rows per wave, four waves' groups
+        // side by side, since a wave each for all of them leaves CUs idle and walks K in dependent
+        // rounds of 17 loads.  Past 2048 big rows one wave takes them all and reads its row once.
+        // 16 x 1024 -> 160: 8.9 -> 3.5 us, -> 2048: 11.4 -> 8.0; 5 x 2048 -> 33: 8.0 -> 4.1.
+        const bool fours = nsmall > 4 && rows <= 2048;
+        const dim3 grid((rows + 3) / 4, fours ? (nsmall + 3) / 4 : 1);
 #define NSOSX_DOT(XDT, PM, JM)                                                                \
     hipLaunchKernelGGL((dot_kernel<XDT, PM, JM>), grid, dim3(256), 0, st, x, inv, w, M, N, K, \
                        magnitude, bias, y, ybf)
-        // (at 2048 rows the wave-per-row form has two workgroups per CU)
-#define NSOSX_DOT_J(XDT, PM)                                                 \
-    if (nsmall > 4 && rows <= 2048)                                          \
-        hipLaunchKernelGGL((dot_split_kernel<XDT, PM>), dim3(rows), dim3(256), 0, st, x, inv, w, M, N, K, \
-                           magnitude, bias, y, ybf);                         \
-    else if (nsmall == 1) NSOSX_DOT(XDT, PM, 1);                                  \
-    else if (nsmall <= 4) NSOSX_DOT(XDT, PM, 4);                             \
+#define NSOSX_DOT_J(XDT, PM)                      \
+    if (nsmall == 1) NSOSX_DOT(XDT, PM, 1);       \
+    else if (nsmall <= 4 || fours) NSOSX_DOT(XDT, PM, 4); \
     else NSOSX_DOT(XDT, PM, kDotMax);
         if (x_dtype == NSOSX_F32) {
             if (per_m) { NSOSX_DOT_J(NSOSX_F32, true) } else { NSOSX_DOT_J(NSOSX_F32, false) }

@@ -3,7 +3,8 @@
 The block quantizes the scan's output for its out_proj, so a last-bit change in the B / C / dt
 projections or in the scan moves int8 codes, which is 2e-4 of the block's output: more than its
 rounding, and what a saved activation or a resumed run would see.  The digests are those of the
-float32 MFMA projections and the recurrence; a kernel that sums in another order fails here.  Inputs come from numpy's generator alone.
+float32 MFMA projections, of the lane chains of few rows and of the recurrence; a kernel that sums
+in another order fails here.  Inputs come from numpy's generator alone.
 """
 import hashlib
 
@@ -24,6 +25,10 @@ LINEAR = {  # m, k, n, input dtype, rms
     (10300, 264, 33, "f32", False): "db4f4f5ae48f67d9",
     (10300, 264, 64, "bf16", False): "2dbca9a6153b709c",
     (1500, 1024, 8, "f32", True): "2ea4bc44904a327a",
+    (16, 1024, 160, "f32", False): "e1da4597b0e72f65",
+    (5, 260, 70, "bf16", True): "9aeae8a526f57bde",
+    (13, 2052, 160, "f32", False): "188e0f3307ab9f52",
+    (9, 512, 2048, "bf16", False): "c34c21016c19cd3e",
 }
 BLOCK = {  # lengths, heads, d_state, dtype
     ((300, 1025), 16, 64, "f32"): "902fcd8100bd1db6",
