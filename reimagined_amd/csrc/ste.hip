@@ -14,6 +14,7 @@
 // longer ones), a forward and backward step 1062 -> 273 us.
 #include "row_sum.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace nsosx {
@@ -42,6 +43,7 @@ struct SteArgs {
     float* dbias;            // [N] or null
     float ws, clip;
     int M, K, N, Mp, Np;
+    int first;               // tile of the launch's first workgroup
 };
 
 // 16-byte chunk c (8 reduction elements) of tile row r: swizzled so that the 16 rows
@@ -306,6 +308,7 @@ __global__ __launch_bounds__(kSteThreads, 2) void ste_gemm_kernel(SteArgs g) {
     const int per = total / 8;
     int t = blockIdx.x;
     if (t < per * 8) t = (t % 8) * per + t / 8;
+    t += g.first;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 2, wn = wave & 3;
@@ -427,6 +430,12 @@ __global__ __launch_bounds__(256) void ste_dmag_kernel(SteArgs g, const int8_t* 
         if (odd != 0.0f) s = odd;  // (only finite gradients: their sum overflowed, s stands)
     }
     dmag[j] = s;
+}
+
+// A copy of an input that an output lies over.
+__global__ __launch_bounds__(256) void ste_copy_kernel(const float* __restrict__ src, int64_t n,
+                                                       float* __restrict__ dst) {
+    for (int64_t i = blockIdx.x * 256LL + threadIdx.x; i < n; i += gridDim.x * 256LL) dst[i] = src[i];
 }
 
 // The exact operands, reduction-contiguous in bf16: qT[k][i] = q[i][k] and tT[k][j] =
@@ -563,6 +572,8 @@ struct SteWorkspace {
     float* dact;      // [M, K] (rms_input only)
     float* inv;       // [M] (rms_input only)
     float* part;      // [4 * K tiles, N]
+    float* grad;      // [M, N], only where an output lies over grad
+    float* mag;       // [N], only where an output lies over magnitude
     int Mp, Np;
     int64_t bytes;
 };
@@ -582,6 +593,8 @@ static SteWorkspace ste_layout(void* base, int M, int K, int N, int rms_input) {
     w.dact = rms_input ? reinterpret_cast<float*>(take(4 * (int64_t)M * K)) : nullptr;
     w.inv = rms_input ? reinterpret_cast<float*>(take(4 * (int64_t)M)) : nullptr;
     w.part = reinterpret_cast<float*>(take(16 * (int64_t)((K + kTC - 1) / kTC) * N));
+    w.grad = reinterpret_cast<float*>(take(4 * (int64_t)M * N));
+    w.mag = reinterpret_cast<float*>(take(4 * (int64_t)N));
     w.bytes = off;
     return w;
 }
@@ -632,19 +645,45 @@ extern "C" int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const in
 
     hipLaunchKernelGGL(ste_pack_kernel, dim3(qblocks + tblocks, (K + 511) / 512), dim3(256), 0, st,
                        q, packed, M, K, N, ws.Mp, ws.Np, ws.qT, ws.tT, qblocks);
+    // The tiles of one launch store while others read.  An output over grad or magnitude makes them
+    // read a copy; dx over the codes, their scales or the latent weights, which only dW's tiles
+    // read, is stored by a launch after those.  (With rms_input dx is the last kernel's.)
+    auto meets = [&](const void* in, int64_t bytes) {
+        auto hit = [&](const float* out, int64_t n) { return out && overlaps(out, 4 * n, in, bytes); };
+        return (!rms_input && hit(dx, (int64_t)M * K)) || hit(dW, (int64_t)N * K) || hit(dmag, N) ||
+               hit(dbias, N);
+    };
+    auto copy = [&](const float* src, int64_t n, float* dst) -> const float* {
+        hipLaunchKernelGGL(ste_copy_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 16384)),
+                           dim3(256), 0, st, src, n, dst);
+        return dst;
+    };
+    const float* gsrc = meets(grad, 4 * (int64_t)M * N) ? copy(grad, (int64_t)M * N, ws.grad) : grad;
+    const float* msrc = magnitude && meets(magnitude, 4 * (int64_t)N) ? copy(magnitude, N, ws.mag) : magnitude;
+    const bool dx_last = !rms_input && (overlaps(dx, 4 * (int64_t)M * K, q, (int64_t)M * K) ||
+                                        overlaps(dx, 4 * (int64_t)M * K, act_scale, 4 * (int64_t)M) ||
+                                        overlaps(dx, 4 * (int64_t)M * K, w_latent, 4 * (int64_t)N * K));
+
     // dW = gp^T @ (x_q * act_scale), zero where |W / (ws + 1e-8f)| > 1 (bitlinear.cpp:1293-1321),
     // with gp = grad * magnitude taken as magnitude[j] * (grad^T @ ...); d_act = gp @ (ternary *
     // weight_scale) (1340); the column sums behind dmag and dbias (1267-1290) on the way
     SteArgs g{};
-    g.grad = grad; g.mag = magnitude; g.as = act_scale; g.qT = ws.qT; g.tT = ws.tT;
+    g.grad = gsrc; g.mag = msrc; g.as = act_scale; g.qT = ws.qT; g.tT = ws.tT;
     g.packed = packed; g.wlat = w_latent; g.dW = dW; g.dact = rms_input ? ws.dact : dx;
     g.part_mag = dmag ? ws.part : nullptr; g.dbias = dbias;
     g.ws = weight_scale; g.clip = weight_scale + 1e-8f;
     g.M = M; g.K = K; g.N = N; g.Mp = ws.Mp; g.Np = ws.Np;
-    hipLaunchKernelGGL(ste_gemm_kernel, dim3((unsigned)tiles), dim3(kSteThreads), kSteSmem, st, g);
+    const int64_t tiles_w = (int64_t)(N + kTR - 1) / kTR * tk;
+    hipLaunchKernelGGL(ste_gemm_kernel, dim3((unsigned)(dx_last ? tiles_w : tiles)), dim3(kSteThreads),
+                       kSteSmem, st, g);
     if (dmag)
         hipLaunchKernelGGL(ste_dmag_kernel, dim3((N + 255) / 256), dim3(256), 0, st, g, q, 4 * tk,
                            dmag);
+    if (dx_last) {
+        g.first = (int)tiles_w;
+        hipLaunchKernelGGL(ste_gemm_kernel, dim3((unsigned)(tiles - tiles_w)), dim3(kSteThreads), kSteSmem,
+                           st, g);
+    }
 
     // dx = rmsnorm_backward(x, d_act, x_norm) (bitlinear.cpp:1352-1355)
     if (rms_input) {

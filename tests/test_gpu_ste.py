@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from reimagined_amd import ops
+from reimagined_amd._lib import call, lib
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
@@ -84,3 +85,42 @@ def test_ste_infinities_and_nan_stay_where_they_are(dev, m, n):
         inf = np.isinf(want[key])
         np.testing.assert_array_equal(g[inf], want[key][inf].astype(np.float32), err_msg=key)
         assert np.array_equal(np.isinf(g), inf), key
+
+
+@pytest.mark.parametrize("m,k,n,out,over", [
+    (300, 384, 384, "dx", "grad"), (384, 272, 384, "dW", "grad"), (256, 528, 260, "dW", "grad"),
+    (300, 272, 260, "dbias", "grad"), (300, 272, 260, "dmag", "grad"),
+    (300, 272, 260, "dbias", "mag"), (300, 272, 260, "dmag", "mag"), (300, 528, 260, "dx", "mag"),
+    (300, 528, 260, "dW", "mag"), (384, 272, 384, "dx", "w"), (300, 272, 260, "dx", "q"),
+    (300, 272, 260, "dx", "s"), (300, 272, 260, "dW", "w")])
+@pytest.mark.parametrize("odd", [False, True])
+def test_ste_outputs_over_inputs(dev, m, k, n, out, over, odd):
+    """An output laid over an input gives the bits of one apart, also where gradients are not finite
+    (dmag reads them again then)."""
+    w, packed, ws, _, x, q, s, grad, mag = _case(dev, m, k, n, True, m + k + n)
+    if odd:
+        grad[3, 5], grad[40, 6], grad[m - 1, n - 1] = np.inf, -np.inf, np.nan
+    t = lambda a: torch.from_numpy(a).to(dev)
+    nbytes = int(lib().nsosx_bitlinear_ste_backward_workspace(m, k, n, 0))
+
+    def run(lay):
+        shapes = {"dx": (m, k), "dW": (n, k), "dmag": (n,), "dbias": (n,)}
+        src = {"q": q.contiguous(), "s": s.contiguous(), "w": t(w), "grad": t(grad), "mag": t(mag)}
+        bufs = {key: torch.empty(shape, device=dev) for key, shape in shapes.items()}
+        if lay:  # one block of memory that holds both from its first byte
+            a, b = src[over], bufs[out]
+            block = torch.empty(max(a.numel() * a.element_size(), b.numel() * 4), dtype=torch.uint8, device=dev)
+            src[over] = block[:a.numel() * a.element_size()].view(a.dtype).view(a.shape).copy_(a)
+            bufs[out] = block[:b.numel() * 4].view(torch.float32).view(b.shape)
+        p = lambda v: v.data_ptr()
+        work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        call("nsosx_bitlinear_ste_backward", None, 0, p(src["q"]), p(src["s"]), p(src["w"]),
+             p(packed_t), float(ws), m, k, n, 0, p(src["mag"]), p(src["grad"]), p(bufs["dx"]), p(bufs["dW"]),
+             p(bufs["dmag"]), p(bufs["dbias"]), p(work), None)
+        torch.cuda.synchronize()
+        return bufs
+
+    packed_t = t(packed.view(np.int32))
+    want, got = run(False), run(True)
+    for key in want:
+        np.testing.assert_array_equal(got[key].cpu().numpy(), want[key].cpu().numpy(), err_msg=key)
