@@ -405,31 +405,64 @@ __global__ __launch_bounds__(kSteThreads, 2) void ste_gemm_kernel(SteArgs g) {
 // dmag[j] = sum_i grad[i][j] * pre[i][j] with pre = acc * (as * ws), taken as
 // ws * sum_k T[j][k] G[j][k] from the dW tiles' G = sum_i grad * as * q.  Where that is
 // not finite, a gradient was not (0 * inf in a row's other products would leave a NaN
-// in place of an infinity): the rows whose gradient is not finite are summed from their
-// own dot products, as the definition has them.
+// in place of an infinity): the rows whose gradient (or scale) is not finite are summed from their
+// own dot products, as the definition has them, by a wave per such column, up to the first NaN
+// (which the sum then stays).  Gradients that overflowed everywhere, 512 x 256 x 256: 15000 us
+// with a thread per column and no end at the NaN, now 66 to 104.
+constexpr int kDmagCols = 32;  // columns per workgroup
+
 __global__ __launch_bounds__(256) void ste_dmag_kernel(SteArgs g, const int8_t* __restrict__ q,
                                                        int parts, float* __restrict__ dmag) {
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= g.N) return;
-    float s = 0.0f;
+    __shared__ float s_sum[kDmagCols];
+    const int j0 = blockIdx.x * kDmagCols;
+    const int tid = threadIdx.x;
+    const float inf = __builtin_inff();
+    if (tid < kDmagCols) {
+        const int j = j0 + tid;
+        float s = 0.0f;
+        if (j < g.N) {
 #pragma unroll 8
-    for (int c = 0; c < parts; ++c) s = __fadd_rn(s, g.part_mag[(int64_t)c * g.N + j]);
-    s = __fmul_rn(s, g.ws);
-    if (!(fabsf(s) < __builtin_inff())) {
-        float odd = 0.0f;
-        for (int i = 0; i < g.M; ++i) {
-            const float gr = g.grad[(int64_t)i * g.N + j];
-            if (fabsf(gr) < __builtin_inff()) continue;
-            int acc = 0;
-            for (int k = 0; k < g.K; ++k) {
-                const uint32_t c = (g.packed[((int64_t)j * g.K + k) >> 4] >> (2 * (k & 15))) & 3u;
-                acc += (c == 0u ? -1 : (c == 2u ? 1 : 0)) * q[(int64_t)i * g.K + k];
-            }
-            odd += gr * (static_cast<float>(acc) * (g.as[i] * g.ws));
+            for (int c = 0; c < parts; ++c) s = __fadd_rn(s, g.part_mag[(int64_t)c * g.N + j]);
+            s = __fmul_rn(s, g.ws);
+            if (fabsf(s) < inf) dmag[j] = s;
         }
-        if (odd != 0.0f) s = odd;  // (only finite gradients: their sum overflowed, s stands)
+        s_sum[tid] = s;
     }
-    dmag[j] = s;
+    __syncthreads();
+    const int lane = tid & 63;
+    for (int c = tid >> 6; c < kDmagCols; c += 4) {
+        const float s = s_sum[c];
+        if (fabsf(s) < inf) continue;
+        const int j = j0 + c;
+        float odd = 0.0f;
+        for (int i0 = 0; i0 < g.M && odd == odd; i0 += 64) {
+            const int i = min(i0 + lane, g.M - 1);
+            const float gr = g.grad[(int64_t)i * g.N + j];
+            const float comb = __fmul_rn(g.as[i], g.ws);
+            unsigned long long rows =
+                __ballot(i0 + lane < g.M && !(fabsf(gr) < inf && fabsf(comb) < inf));
+            while (rows && odd == odd) {
+                const int l = __builtin_ctzll(rows);
+                rows &= rows - 1;
+                int acc = 0;
+                for (int k = 16 * lane; k < g.K; k += 16 * 64) {  // K % 16 == 0
+                    const uint32_t w = g.packed[((int64_t)j * g.K + k) >> 4];
+                    const int4 x = *reinterpret_cast<const int4*>(q + (int64_t)(i0 + l) * g.K + k);
+                    const int xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const uint32_t code = (w >> (2 * e)) & 3u;
+                        acc += (code == 0u ? -1 : (code == 2u ? 1 : 0)) *
+                               static_cast<int8_t>(xs[e >> 2] >> (8 * (e & 3)));
+                    }
+                }
+                acc = wave_sum_i32(acc);
+                odd += __shfl(gr, l) * (static_cast<float>(acc) * __shfl(comb, l));
+            }
+        }
+        // (only finite gradients: their sum overflowed, s stands)
+        if (lane == 0) dmag[j] = odd != 0.0f ? odd : s;
+    }
 }
 
 // A copy of an input that an output lies over.
@@ -677,8 +710,8 @@ extern "C" int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const in
     hipLaunchKernelGGL(ste_gemm_kernel, dim3((unsigned)(dx_last ? tiles_w : tiles)), dim3(kSteThreads),
                        kSteSmem, st, g);
     if (dmag)
-        hipLaunchKernelGGL(ste_dmag_kernel, dim3((N + 255) / 256), dim3(256), 0, st, g, q, 4 * tk,
-                           dmag);
+        hipLaunchKernelGGL(ste_dmag_kernel, dim3((N + kDmagCols - 1) / kDmagCols), dim3(256), 0, st, g, q,
+                           4 * tk, dmag);
     if (dx_last) {
         g.first = (int)tiles_w;
         hipLaunchKernelGGL(ste_gemm_kernel, dim3((unsigned)(tiles - tiles_w)), dim3(kSteThreads), kSteSmem,

@@ -124,3 +124,45 @@ def test_ste_outputs_over_inputs(dev, m, k, n, out, over, odd):
     want, got = run(False), run(True)
     for key in want:
         np.testing.assert_array_equal(got[key].cpu().numpy(), want[key].cpu().numpy(), err_msg=key)
+
+
+def test_ste_dmag_with_row_scales_not_finite(dev):
+    """A row whose act_scale is infinite or NaN leaves in dmag what the definition gives."""
+    m, k, n = 70, 272, 40
+    c = list(_case(dev, m, k, n, True, 5))
+    c[6] = c[6].clone()
+    c[6][3], c[6][69] = np.inf, np.inf
+    got, want = _run(dev, c)["dmag"], _want(c)["dmag"]
+    np.testing.assert_array_equal(got, want.astype(np.float32))
+    assert np.isinf(got).any()
+    c[6][5] = np.nan
+    assert np.isnan(_run(dev, c)["dmag"]).all()
+
+
+@pytest.mark.parametrize("kind", ["+inf", "inf", "nan"])
+def test_ste_time_when_every_gradient_overflowed(dev, kind):
+    """A step whose gradients overflowed (as under loss scaling) takes about its usual time: the
+    tiles' second pass over the infinities and a short walk per column, not M * K steps of one
+    thread (290 times the usual time at a quarter of this size)."""
+    m, k, n = 1024, 512, 512
+    w, packed, ws, _, x, q, s, grad, mag = _case(dev, m, k, n, True, 11)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    wd, pd, md = t(w), t(packed.view(np.int32)), t(mag)
+    usual = t(grad)
+    bad = {"+inf": torch.full_like(usual, np.inf), "nan": torch.full_like(usual, np.nan),
+           "inf": torch.where(usual > 0, np.inf, -np.inf).to(torch.float32)}[kind]
+
+    def us(g):
+        run = lambda: ops.bitlinear_ste_backward(x, q, s, wd, pd, float(ws), g, False, md, True)
+        run()
+        best = np.inf
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            run()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    assert us(bad) < 10 * us(usual)
