@@ -4,7 +4,8 @@
 // Both contractions have one f32 operand (the gradient) and one operand that bf16
 // holds exactly: the int8 codes (|q| <= 127, 7 bits) and the ternary weights.  The
 // f32 operand is cut into three bf16 pieces (8 + 8 + 8 significant bits: their sum
-// is the value), so three v_mfma_f32_32x32x16_bf16 with f32 accumulation give the
+// is the value, of denormals too, since 2^24 times the operand is cut: the matrix cores
+// read a denormal bf16 as zero), so three v_mfma_f32_32x32x16_bf16 with f32 accumulation give the
 // products that v_mfma_f32_32x32x2_f32 gives, each exact before it is added, at a
 // sixteenth of the matrix-core time per pass.  Before: two fp32-MFMA GEMMs at the
 // card's fp32 rate (400 + 407 us at M = 4096, K = 1024, N = 4096), a full ternary
@@ -29,10 +30,16 @@ constexpr int kPlane = kTR * kTK * 2;         // bytes of one gradient piece of 
 constexpr int kSteStage = 3 * kPlane + kTC * kTK * 2;
 constexpr int kSteSmem = 2 * kSteStage;       // double buffered: 80 KB
 
+// The gradient operand is cut at 2^24 times its value, where the last bit of the smallest
+// float (2^-149) is a normal bf16; the sums are taken back by as much.
+constexpr float kSteUp = 16777216.0f;
+
 struct SteArgs {
     const float* grad;       // [M, N]
     const float* mag;        // [N] or null
     const float* as;         // [M]
+    const float* as_up;      // [M]: as * kSteUp
+    const float* mag_up;     // [N]: mag * kSteUp
     const uint16_t* qT;      // bf16 [K][Mp]: the codes, reduction-contiguous, zero past M
     const uint16_t* tT;      // bf16 [K][Np]: the ternary weights, zero past N
     const uint32_t* packed;  // [N, K / 16]
@@ -75,7 +82,8 @@ __device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t& hi, ui
 // elements of one tile row per stage.  The whole stages run branch-free (rows and columns
 // past the operands re-read the last: their outputs are never stored), the split's VALU
 // between the MFMAs and the loads two stages ahead; a last stage cut by the reduction's
-// end, and a tile that meets an infinity, go through slow_stage().
+// end goes through slow_stage().  So does, from the start and without the factor 2^24, a tile
+// with an output that is not finite: an operand was not, or only the factor overflowed.
 // colsum (DW): the thread's share of sum_i grad[i][j] for its column.
 template <bool DW, bool MAG>
 __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char* smem,
@@ -116,14 +124,13 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
             const float* p = asrc + (int64_t)n * g.N;
 #pragma unroll
             for (int e = 0; e < 8; ++e) s.f[e] = p[(int64_t)e * g.N];
-            __builtin_memcpy(s.sc, g.as + n, 32);  // (4-byte aligned)
+            __builtin_memcpy(s.sc, g.as_up + n, 32);  // (4-byte aligned)
         } else {
             __builtin_memcpy(s.f, asrc + n, 32);
-            if (MAG) __builtin_memcpy(s.sc, g.mag + n, 32);
+            if (MAG) __builtin_memcpy(s.sc, g.mag_up + n, 32);
         }
     };
     const int a_at = tile_at(row, chunk);
-    float top = 0.0f;
     auto put = [&](char* dst, const u32x4 (&piece)[3]) {
 #pragma unroll
         for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dst + p * kPlane + a_at) = piece[p];
@@ -134,9 +141,8 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
             *reinterpret_cast<u32x4*>(dst + 3 * kPlane + tile_at((tid >> 2) + 128 * i, tid & 3)) = s.b[i];
     };
     auto cut = [&](const Stage& s, int p, u32x4 (&piece)[3]) {  // elements 2p, 2p + 1
-        const float v0 = DW || MAG ? __fmul_rn(s.f[2 * p], s.sc[2 * p]) : s.f[2 * p];
-        const float v1 = DW || MAG ? __fmul_rn(s.f[2 * p + 1], s.sc[2 * p + 1]) : s.f[2 * p + 1];
-        top = fmaxf(top, fmaxf(fabsf(v0), fabsf(v1)));
+        const float v0 = __fmul_rn(s.f[2 * p], DW || MAG ? s.sc[2 * p] : kSteUp);
+        const float v1 = __fmul_rn(s.f[2 * p + 1], DW || MAG ? s.sc[2 * p + 1] : kSteUp);
         uint32_t h, m, l;
         split3_pair<false>(v0, v1, h, m, l);
         piece[0][p] = h; piece[1][p] = m; piece[2][p] = l;
@@ -207,7 +213,7 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
         load(st + 3, s);
         fence();
     };
-    auto slow_stage = [&](int st, bool cols) {
+    auto slow_stage = [&](int st, bool up) {  // up: times 2^24, and the columns' sums
         Stage s;
         const int n = st * kTK + chunk * 8;
         float v[8];
@@ -215,12 +221,12 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
         for (int e = 0; e < 8; ++e) {
             const int at = min(n + e, red - 1);
             const float f = asrc[DW ? (int64_t)at * g.N : (int64_t)at];
-            const float sc = DW ? g.as[at] : (MAG ? g.mag[at] : 1.0f);
+            const float sc = DW ? (up ? g.as_up : g.as)[at]
+                                : (MAG ? (up ? g.mag_up : g.mag)[at] : (up ? kSteUp : 1.0f));
             s.f[e] = n + e < red ? f : 0.0f;
             v[e] = n + e < red ? __fmul_rn(f, sc) : 0.0f;
-            top = fmaxf(top, fabsf(v[e]));
         }
-        if (DW) add_cols(s, cols);
+        if (DW) add_cols(s, up);
 #pragma unroll
         for (int i = 0; i < 2; ++i) s.b[i] = *reinterpret_cast<const u32x4*>(bsrc[i] + st * kTK);
         u32x4 piece[3];
@@ -284,17 +290,26 @@ __device__ __forceinline__ void ste_tile(const SteArgs& g, int o0, int k0, char*
         __syncthreads();  // (the stage past the end was read, though not used)
     }
     if (full * kTK < red) slow_stage(full, true);
-    if (__syncthreads_or(top == __builtin_inff())) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int n = 0; n < 2; ++n) acc[i][n] = total[i][n] = v16f{};
-        for (int st = 0; st * kTK < red; ++st) slow_stage(st, false);
-    }
+    bool odd = false;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int n = 0; n < 2; ++n) total[i][n] += acc[i][n];
+        for (int n = 0; n < 2; ++n) {
+            total[i][n] = (total[i][n] + acc[i][n]) * (1.0f / kSteUp);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) odd |= !(fabsf(total[i][n][r]) < __builtin_inff());
+        }
+    if (__syncthreads_or(odd)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) acc[i][n] = v16f{};
+        for (int st = 0; st * kTK < red; ++st) slow_stage(st, false);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) total[i][n] = acc[i][n];
+    }
 }
 
 // dW and d_act tiles in one launch (each alone is 128 tiles at 4096 x 1024, together one
@@ -474,17 +489,24 @@ __global__ __launch_bounds__(256) void ste_copy_kernel(const float* __restrict__
 // The exact operands, reduction-contiguous in bf16: qT[k][i] = q[i][k] and tT[k][j] =
 // T[j][k], zero in the padding columns up to a multiple of 32.  A thread takes 16 k of
 // 8 rows and writes, per k, its 8 rows as 16 bytes (a k row's 64 columns of a workgroup
-// are one 128-byte line).
+// are one 128-byte line).  And the factors of the gradient operand, times kSteUp.
 __global__ __launch_bounds__(256) void ste_pack_kernel(const int8_t* __restrict__ q,
                                                        const uint32_t* __restrict__ packed, int M,
                                                        int K, int N, int Mp, int Np,
                                                        uint16_t* __restrict__ qT,
-                                                       uint16_t* __restrict__ tT, int qblocks) {
+                                                       uint16_t* __restrict__ tT, int qblocks,
+                                                       const float* __restrict__ as,
+                                                       const float* __restrict__ mag,
+                                                       float* __restrict__ as_up,
+                                                       float* __restrict__ mag_up) {
     const bool codes = (int)blockIdx.x < qblocks;
     const int r0 = ((codes ? blockIdx.x : blockIdx.x - qblocks) * 8 + (threadIdx.x & 7)) * 8;
     const int k0 = (blockIdx.y * 32 + (threadIdx.x >> 3)) * 16;
     const int rows = codes ? M : N, pad = codes ? Mp : Np;
     if (k0 >= K || r0 >= pad) return;  // pad % 8 == 0, K % 16 == 0
+    const float* factor = codes ? as : mag;
+    if (k0 == 0 && factor)
+        for (int r = r0; r < min(r0 + 8, rows); ++r) (codes ? as_up : mag_up)[r] = factor[r] * kSteUp;
     uint16_t v[16][8];
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
@@ -607,6 +629,8 @@ struct SteWorkspace {
     float* part;      // [4 * K tiles, N]
     float* grad;      // [M, N], only where an output lies over grad
     float* mag;       // [N], only where an output lies over magnitude
+    float* as_up;     // [M]
+    float* mag_up;    // [N]
     int Mp, Np;
     int64_t bytes;
 };
@@ -628,6 +652,8 @@ static SteWorkspace ste_layout(void* base, int M, int K, int N, int rms_input) {
     w.part = reinterpret_cast<float*>(take(16 * (int64_t)((K + kTC - 1) / kTC) * N));
     w.grad = reinterpret_cast<float*>(take(4 * (int64_t)M * N));
     w.mag = reinterpret_cast<float*>(take(4 * (int64_t)N));
+    w.as_up = reinterpret_cast<float*>(take(4 * (int64_t)M));
+    w.mag_up = reinterpret_cast<float*>(take(4 * (int64_t)N));
     w.bytes = off;
     return w;
 }
@@ -677,7 +703,8 @@ extern "C" int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const in
         return fail(NSOSX_ERR_OVERFLOW, "bitlinear_ste_backward: size too large");
 
     hipLaunchKernelGGL(ste_pack_kernel, dim3(qblocks + tblocks, (K + 511) / 512), dim3(256), 0, st,
-                       q, packed, M, K, N, ws.Mp, ws.Np, ws.qT, ws.tT, qblocks);
+                       q, packed, M, K, N, ws.Mp, ws.Np, ws.qT, ws.tT, qblocks, act_scale, magnitude,
+                       ws.as_up, ws.mag_up);
     // The tiles of one launch store while others read.  An output over grad or magnitude makes them
     // read a copy; dx over the codes, their scales or the latent weights, which only dW's tiles
     // read, is stored by a launch after those.  (With rms_input dx is the last kernel's.)
@@ -701,7 +728,7 @@ extern "C" int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const in
     // with gp = grad * magnitude taken as magnitude[j] * (grad^T @ ...); d_act = gp @ (ternary *
     // weight_scale) (1340); the column sums behind dmag and dbias (1267-1290) on the way
     SteArgs g{};
-    g.grad = gsrc; g.mag = msrc; g.as = act_scale; g.qT = ws.qT; g.tT = ws.tT;
+    g.grad = gsrc; g.mag = msrc; g.as = act_scale; g.as_up = ws.as_up; g.mag_up = ws.mag_up; g.qT = ws.qT; g.tT = ws.tT;
     g.packed = packed; g.wlat = w_latent; g.dW = dW; g.dact = rms_input ? ws.dact : dx;
     g.part_mag = dmag ? ws.part : nullptr; g.dbias = dbias;
     g.ws = weight_scale; g.clip = weight_scale + 1e-8f;

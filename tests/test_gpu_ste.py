@@ -166,3 +166,28 @@ def test_ste_time_when_every_gradient_overflowed(dev, kind):
         return best
 
     assert us(bad) < 10 * us(usual)
+
+
+@pytest.mark.parametrize("e", [-126, -118, -110, -100, 0, 60, 84])
+@pytest.mark.parametrize("with_mag", [True, False])
+def test_ste_precision_at_every_magnitude(dev, with_mag, e):
+    """Gradients of 2^e: their pieces hold every bit, of small ones too (a denormal bf16 reads as
+    zero in the matrix cores), and sums that overflow only on the way come out as they are.  The
+    bound is the float sum's, as above; results below 2^-126 round to multiples of 2^-149."""
+    m, k, n = 200, 272, 132
+    c = list(_case(dev, m, k, n, with_mag, 17, spread=16.0))
+    with np.errstate(under="ignore"):
+        c[7] = np.ldexp(c[7], e).astype(np.float32)
+    c[6] = torch.full_like(c[6], 2.0 ** 12)  # (keeps dW and dmag normal for the smallest)
+    got, want = _run(dev, tuple(c)), _want(tuple(c))
+    absw = list(c)
+    absw[7], absw[3], absw[5], absw[0] = np.abs(c[7]), np.abs(c[3]), c[5].abs(), np.zeros_like(c[0])
+    size = _want(tuple(absw))
+    terms = {"dW": m + 4, "dx": n + 4, "dmag": m + k + 8, "dbias": m}
+    if with_mag:
+        a = np.abs(c[5].cpu().numpy().astype(np.float64)) * c[6].cpu().numpy().astype(np.float64)[:, None]
+        size["dmag"] = float(c[2]) * ((np.abs(c[7]).astype(np.float64).T @ a) * np.abs(c[3])).sum(1)
+    for key, g in got.items():
+        err = np.abs(g.astype(np.float64) - want[key])
+        # (a product that underflows is rounded to 2^-149 before it is added)
+        assert np.all(err <= terms[key] * (U * size[key] + 2.0 ** -149)), key
