@@ -588,7 +588,7 @@ __global__ __launch_bounds__(512) void rms_backward_row_kernel(const void* __res
     for (int j = 0; j < 8; ++j) sq[j] = __fmul_rn(v[j], v[j]);
     *reinterpret_cast<float4*>(s_dyn + tid * 8) = make_float4(sq[0], sq[1], sq[2], sq[3]);
     *reinterpret_cast<float4*>(s_dyn + tid * 8 + 4) = make_float4(sq[4], sq[5], sq[6], sq[7]);
-    const float sum = row_sum_in_order<8>(sq, blockDim.x >> 6, s_dyn, reinterpret_cast<SumRun*>(s_dyn + 8 * blockDim.x),
+    const float sum = row_sum_in_order<8>(sq, K, blockDim.x >> 6, s_dyn, reinterpret_cast<SumRun*>(s_dyn + 8 * blockDim.x),
                                        s_w, s_mask);
     if (tid == 0)
         s_inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, static_cast<float>(K)), eps)));
