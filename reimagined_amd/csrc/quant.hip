@@ -290,15 +290,22 @@ __global__ __launch_bounds__(256) void rms_inv_small_kernel(const void* __restri
 // VEC: K % 8 == 0, every row 16-byte aligned -> 8 elements per lane-load,
 // the row kept in registers between the two passes when K <= 4096.
 // ===========================================================================
+
 // ===========================================================================
 // RMS_PERI + codes in one launch, a workgroup per row (row_sum.hpp takes the in-order sum;
 // by one lane walking the row from LDS it was 4.2 us of a call at K = 1024 and 16 us at 4096).
 // Time per call, us, before (a serial sum up to 1024 rows, two passes above) -> now:
-//   bf16   1 x 1024 6.4 -> 5.0    64 x 2048 11.4 -> 6.4    1024 x 4096 32.8 -> 11.6
-//   f32  300 x 768  6.8 -> 5.7  1500 x 2048 18.2 -> 9.6    3000 x 4096 38.8 -> 27.4
+//   bf16   1 x 1024 6.2 -> 5.0    64 x 2048 11.2 -> 6.5    1000 x 4096 32.6 -> 11.5
+//   f32   64 x 768  5.7 -> 5.2  1600 x 2048 18.7 -> 10.3   3000 x 4096 39.1 -> 28.2
 // It is bound by instruction issue (about 1000 per 1024-element row, half of them the walk),
-// so past 3072 rows of bf16 the two streaming passes, a lane per row, are the faster ones
-// (4096 x 2048: 17.2 against 18.5 us), and past 6144 rows of f32 (4096 where K < 1024).
+// so for many rows the two streaming passes, a lane per row, are the faster ones.
+//
+// Rows up to which the one launch is taken, from two passes / one launch at K 64 .. 4096, us:
+//   bf16  3000 rows: K 768 11.9 / 8.6, 2048 16.4 / 15.5, 2560 20.6 / 21.2, 3584 27.9 / 26.4;
+//         2600: K 2560 20.0 / 19.7; 3400: K 1024 10.2 / 10.9
+//   f32   3400 rows: K 1280 14.6 / 14.0, 3072 29.6 / 28.4; 4200: 15.8 / 16.1, 31.2 / 32.7;
+//         a power of two, whose rows the lanes of the RMS pass find on the same channels, 6000:
+//         K 1024 16.9 / 15.6, 2048 27.9 / 25.5, 4096 55.0 / 49.9
 // ===========================================================================
 template <int DT>
 __global__ __launch_bounds__(512) void quantize_row_rms_kernel(const void* __restrict__ x, int K,
@@ -540,12 +547,19 @@ void launch_rms_inv(const void* x, int dtype, int M, int K, float eps, float* in
     else launch_rms_inv_t<NSOSX_BF16>(x, M, K, eps, inv, st);
 }
 
+// Rows up to which RMS_PERI and the codes are one launch (measured at quantize_row_rms_kernel).
+static int one_launch_rows(int dtype, int K) {
+    if (dtype == NSOSX_BF16) return K <= 2048 ? 3072 : 2560;
+    if (K < 1024) return 4096;
+    return (K & (K - 1)) == 0 ? 6144 : 3584;
+}
+
 template <int DT>
 static int launch_quantize(const void* x, int M, int K, int bits, int rms_input, int8_t* q,
                            float* act_scale, float* rms_ws, hipStream_t st) {
     const float qm = q_max_for_bits(bits);
     const int elem = DT == NSOSX_F32 ? 4 : 2;
-    const int few = DT == NSOSX_BF16 ? 3072 : (K >= 1024 ? 6144 : 4096);
+    const int few = one_launch_rows(DT, K);
     if (rms_input && M <= few && K % 8 == 0 && K <= kQSmallMaxK &&
         reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 8 == 0) {
         const int threads = (K / 8 + 63) / 64 * 64;

@@ -68,6 +68,18 @@ def test_few_rows_equal_many_rows(dev, k):
     np.testing.assert_array_equal(s.cpu().numpy(), ws[:64].cpu().numpy())
 
 
+@pytest.mark.parametrize("bf16,k,rows", [(True, 2048, 3072), (True, 2560, 2560), (False, 896, 4096),
+                                         (False, 1024, 6144), (False, 1280, 3584)])
+def test_last_rows_of_the_one_launch_and_first_of_the_passes(dev, bf16, k, rows):
+    """Both sides of the row limit leave the bits of the rows by themselves."""
+    x = torch.randn((rows + 1, k), device=dev).to(torch.bfloat16 if bf16 else torch.float32)
+    x[-1, : k // 2] = 0
+    want_q, want_s = ops.quantize_activations_bitnet(x[-65:].contiguous(), 8, rms_input=True)
+    for part in (x[1:].contiguous(), x):
+        q, s = ops.quantize_activations_bitnet(part, 8, rms_input=True)
+        assert torch.equal(q[-65:], want_q) and torch.equal(s[-65:], want_s)
+
+
 @pytest.mark.parametrize("k,n", [(64, 48), (512, 33), (1024, 4096), (2048, 1000), (2112, 64),
                                  (4096, 256)])
 @pytest.mark.parametrize("bf16", [True, False])
