@@ -306,6 +306,8 @@ __global__ __launch_bounds__(256) void rms_inv_small_kernel(const void* __restri
 //   f32   3400 rows: K 1280 14.6 / 14.0, 3072 29.6 / 28.4; 4200: 15.8 / 16.1, 31.2 / 32.7;
 //         a power of two, whose rows the lanes of the RMS pass find on the same channels, 6000:
 //         K 1024 16.9 / 15.6, 2048 27.9 / 25.5, 4096 55.0 / 49.9
+//   Rows that are not a multiple of 256 cost the passes up to twice as much: K 2600, 3000 rows
+//   of bf16 42.5 / 24.2, 6000 of f32 76.8 / 44.6.
 // ===========================================================================
 template <int DT>
 __global__ __launch_bounds__(512) void quantize_row_rms_kernel(const void* __restrict__ x, int K,
@@ -549,9 +551,10 @@ void launch_rms_inv(const void* x, int dtype, int M, int K, float eps, float* in
 
 // Rows up to which RMS_PERI and the codes are one launch (measured at quantize_row_rms_kernel).
 static int one_launch_rows(int dtype, int K) {
-    if (dtype == NSOSX_BF16) return K <= 2048 ? 3072 : 2560;
+    const bool even = K % 256 == 0;  // the passes' better case
+    if (dtype == NSOSX_BF16) return even && K > 2048 ? 2560 : 3072;
     if (K < 1024) return 4096;
-    return (K & (K - 1)) == 0 ? 6144 : 3584;
+    return even && (K & (K - 1)) ? 3584 : 6144;
 }
 
 template <int DT>

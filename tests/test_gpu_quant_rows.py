@@ -68,8 +68,8 @@ def test_few_rows_equal_many_rows(dev, k):
     np.testing.assert_array_equal(s.cpu().numpy(), ws[:64].cpu().numpy())
 
 
-@pytest.mark.parametrize("bf16,k,rows", [(True, 2048, 3072), (True, 2560, 2560), (False, 896, 4096),
-                                         (False, 1024, 6144), (False, 1280, 3584)])
+@pytest.mark.parametrize("bf16,k,rows", [(True, 2048, 3072), (True, 2560, 2560), (True, 2600, 3072), (False, 896, 4096),
+                                         (False, 1024, 6144), (False, 1280, 3584), (False, 1288, 6144)])
 def test_last_rows_of_the_one_launch_and_first_of_the_passes(dev, bf16, k, rows):
     """Both sides of the row limit leave the bits of the rows by themselves."""
     x = torch.randn((rows + 1, k), device=dev).to(torch.bfloat16 if bf16 else torch.float32)
