@@ -175,8 +175,8 @@ int nsosx_ternary_gemm_mfma(const int8_t* q, const float* act_scale, const uint3
 
 /* bitnet_gemm_158bit_gpu (include/bitnet_gpu_dispatch.h:46-51,
  * src/bitnet_gpu_dispatch.cpp:65-174): quantize x then ternary GEMM.
- * q_workspace: int8 [M, K]; scale_workspace: f32 [M]: the codes and act_scale
- * after the call; rms_workspace: f32 [M] (only with rms_input; scratch). */
+ * q_workspace: int8 [M, K]; scale_workspace: f32 [M]; rms_workspace: f32 [M]
+ * (only with rms_input): the codes, act_scale and 1 / rms after the call. */
 int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_t* packed,
                             float weight_scale, int M, int K, int N, int precision_bits,
                             int rms_input, const float* magnitude, const float* bias, void* y,

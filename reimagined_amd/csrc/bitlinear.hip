@@ -106,6 +106,17 @@ extern "C" int nsosx_ternary_gemm(const int8_t* q, const float* act_scale, const
 // Widest layer whose one-row forward is one launch.
 constexpr int kRowMaxN = 16384;
 
+// Whether the row, the output and the three workspaces of a one-row forward lie apart: one launch
+// reads the row in every workgroup while the first ones store.
+static bool row_buffers_apart(const void* x, int64_t x_bytes, const void* y, int64_t y_bytes,
+                              const int8_t* q, int K, const float* scale, const float* rms) {
+    const struct { const void* p; int64_t bytes; } b[] = {{x, x_bytes}, {y, y_bytes}, {q, K}, {scale, 4}, {rms, 4}};
+    for (int i = 0; i < 5; ++i)
+        for (int j = 0; j < i; ++j)
+            if (b[i].p && b[j].p && overlaps(b[i].p, b[i].bytes, b[j].p, b[j].bytes)) return false;
+    return true;
+}
+
 extern "C" int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_t* packed,
                                        float weight_scale, int M, int K, int N,
                                        int precision_bits, int rms_input, const float* magnitude,
@@ -118,15 +129,17 @@ extern "C" int nsosx_bitlinear_forward(const void* x, int x_dtype, const uint32_
     if (rc) return rc;
     // one row (decode): both in one launch.  The same argument checks as the two calls make;
     // past a few rounds of workgroups each would quantize again what one launch does once, and
-    // an output written over its own input has to wait until every workgroup has read the row
+    // buffers that lie over one another need the first launch to end before the second begins
     if (M == 1 && x && scale_workspace && (!rms_input || rms_workspace) && precision_bits >= 2 &&
         precision_bits <= 8 && valid_dtype(x_dtype) && K % 64 == 0 && K <= kQSmallMaxK &&
         N <= kRowMaxN && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-        !overlaps(x, (int64_t)K * (x_dtype == NSOSX_F32 ? 4 : 2), y, (int64_t)N * (y_dtype == NSOSX_F32 ? 4 : 2))) {
+        row_buffers_apart(x, (int64_t)K * (x_dtype == NSOSX_F32 ? 4 : 2), y,
+                          (int64_t)N * (y_dtype == NSOSX_F32 ? 4 : 2), q_workspace, K,
+                          scale_workspace, rms_input ? rms_workspace : nullptr)) {
         const float q_max = precision_bits <= 2 ? 1.0f : static_cast<float>((1 << (precision_bits - 1)) - 1);
         const GemvProblem pb{packed, magnitude, bias, weight_scale, N, K};
         launch_bitlinear_row(pb, x, x_dtype, q_max, rms_input != 0, q_workspace, scale_workspace,
-                             y, y_dtype, static_cast<hipStream_t>(stream));
+                             rms_workspace, y, y_dtype, static_cast<hipStream_t>(stream));
         return check_launch("bitlinear_forward");
     }
     rc = nsosx_quantize_act_i8(x, x_dtype, M, K, precision_bits, rms_input, q_workspace,

@@ -74,7 +74,8 @@ void launch_gemv(const GemvProblem& pb, const int8_t* q, const float* as, int M,
                  int y_dtype, int32_t* acc, hipStream_t st);
 // gemv.hip: quantization and GEMV of one row in one launch (K % 64 == 0, K <= kQSmallMaxK)
 void launch_bitlinear_row(const GemvProblem& pb, const void* x, int dtype, float q_max, bool rms,
-                          int8_t* q, float* act_scale, void* y, int y_dtype, hipStream_t st);
+                          int8_t* q, float* act_scale, float* rms_inv, void* y, int y_dtype,
+                          hipStream_t st);
 // skinny.hip: the MFMA decode GEMV (2 <= M <= 32, skinny_ok), on the reference words
 // or (mfma_layout) the MFMA-layout words; and the grouped form for nsosx_grouped_gemv
 bool skinny_ok(int M, int K, int N);

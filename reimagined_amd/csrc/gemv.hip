@@ -369,11 +369,11 @@ __device__ __forceinline__ void quantize_one_row(const void* x, int K, float q_m
 // its waves run the M = 1 GEMV on it.  The quantization's time is the same as in a launch of its
 // own (it is a chain of latencies on one CU), the second launch and the codes' trip through
 // memory are saved: 8.5 -> 7.5 us of GPU time at 1024 -> 4096, and one launch of host time.
-// The first workgroup keeps the codes and their scale for the caller.
+// The first workgroup keeps the codes, their scale and 1 / rms for the caller.
 template <int DT, int YDT, bool RMS>
 __global__ __launch_bounds__(256) void bitlinear_row_kernel(GemvProblem pb, const void* __restrict__ x,
                                                             float q_max, int8_t* q, float* act_scale,
-                                                            void* y) {
+                                                            float* rms_inv, void* y) {
     __shared__ __align__(16) float s_row[RMS ? kQSmallMaxK : 4];
     __shared__ __align__(16) int8_t s_q[kQSmallMaxK];
     __shared__ SumRun s_run[RMS ? 256 : 1];
@@ -384,18 +384,22 @@ __global__ __launch_bounds__(256) void bitlinear_row_kernel(GemvProblem pb, cons
     if (blockIdx.x == 0) {
         for (int i = threadIdx.x * 4; i < pb.K; i += 256 * 4)
             *reinterpret_cast<uint32_t*>(q + i) = *reinterpret_cast<const uint32_t*>(s_q + i);
-        if (threadIdx.x == 0) act_scale[0] = s_scale;
+        if (threadIdx.x == 0) {
+            act_scale[0] = s_scale;
+            if (RMS) rms_inv[0] = scratch.inv;
+        }
     }
     const int wave_id = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     gemv_body_long<1, YDT, false>(pb, s_q, &s_scale, 1, y, nullptr, wave_id, gridDim.x * 4, 1);
 }
 
 void launch_bitlinear_row(const GemvProblem& pb, const void* x, int dtype, float q_max, bool rms,
-                          int8_t* q, float* act_scale, void* y, int y_dtype, hipStream_t st) {
+                          int8_t* q, float* act_scale, float* rms_inv, void* y, int y_dtype,
+                          hipStream_t st) {
     const dim3 grid(gemv_grid(pb.N, pb.K, 1)), block(256);
 #define NSOSX_ROW(DT, YDT)                                                                      \
-    if (rms) hipLaunchKernelGGL((bitlinear_row_kernel<DT, YDT, true>), grid, block, 0, st, pb, x, q_max, q, act_scale, y); \
-    else hipLaunchKernelGGL((bitlinear_row_kernel<DT, YDT, false>), grid, block, 0, st, pb, x, q_max, q, act_scale, y);
+    if (rms) hipLaunchKernelGGL((bitlinear_row_kernel<DT, YDT, true>), grid, block, 0, st, pb, x, q_max, q, act_scale, rms_inv, y); \
+    else hipLaunchKernelGGL((bitlinear_row_kernel<DT, YDT, false>), grid, block, 0, st, pb, x, q_max, q, act_scale, rms_inv, y);
     if (dtype == NSOSX_F32) {
         if (y_dtype == NSOSX_F32) { NSOSX_ROW(NSOSX_F32, NSOSX_F32) } else { NSOSX_ROW(NSOSX_F32, NSOSX_BF16) }
     } else {

@@ -124,6 +124,46 @@ def test_one_row_forward_keeps_the_codes_and_runs_in_place(dev, orc, k, n, rms):
         assert torch.equal(y[:n], want.view(-1))
 
 
+def _one_row_forward(dev, k, n, rms, pk, ws, x, over=None):
+    """The C entry on buffers of its own, or with over = (a, b): b lies over a from its first byte."""
+    size = {"x": 4 * k, "y": 4 * n, "q": k, "s": 4, "r": 4}
+    mem = {key: torch.zeros(max(size.values()), dtype=torch.uint8, device=dev) for key in size}
+    if over:
+        mem[over[1]] = mem[over[0]]
+    mem["x"][:4 * k] = x.view(torch.uint8).view(-1)
+    p = {key: v.data_ptr() for key, v in mem.items()}
+    call("nsosx_bitlinear_forward", p["x"], 0, pk.data_ptr(), ws, 1, k, n, 8, int(rms), None, None,
+         p["y"], 0, p["q"], p["s"], p["r"], None)
+    torch.cuda.synchronize()
+    return {key: v[:size[key]] for key, v in mem.items()}
+
+
+@pytest.mark.parametrize("k,n", [(512, 512), (1024, 1000), (4096, 4096)])
+@pytest.mark.parametrize("rms", [True, False])
+def test_one_row_forward_keeps_codes_scale_and_rms(dev, orc, k, n, rms):
+    """The workspaces hold the row's codes, scale and 1 / rms afterwards, as a backward reads them;
+    buffers that lie over one another leave what one apart from the other leaves."""
+    rng = np.random.default_rng(k)
+    packed, ws, _ = orc.pack_weights(rng.standard_normal((n, k)).astype(np.float32))
+    pk = torch.from_numpy(packed.view(np.int32)).to(dev)
+    x = torch.randn((1, k), device=dev)
+    want = {"q": torch.zeros((1, k), dtype=torch.int8, device=dev), "s": torch.zeros(1, device=dev),
+            "r": torch.zeros(1, device=dev)}
+    call("nsosx_quantize_act_i8", x.data_ptr(), 0, 1, k, 8, int(rms), want["q"].data_ptr(),
+         want["s"].data_ptr(), want["r"].data_ptr(), None)
+    want["y"] = ops.ternary_gemm(want["q"], want["s"], pk, ws, n)
+    want = {key: v.contiguous().view(torch.uint8).view(-1) for key, v in want.items()}
+    got = _one_row_forward(dev, k, n, rms, pk, ws, x)
+    for key in want:
+        assert torch.equal(got[key], want[key]), key
+    # the later of two stores stands: r, then s, then q, then y
+    for a, b in (("x", "y"), ("x", "q"), ("x", "s"), ("x", "r"), ("r", "s"), ("r", "y"), ("r", "q")):
+        got = _one_row_forward(dev, k, n, rms, pk, ws, x, (a, b))
+        for key in ("y", "q", "s", "r"):
+            if not (key == "r" and (a == "r" or not rms)):
+                assert torch.equal(got[key], want[key]), (a, b, key)
+
+
 @pytest.mark.parametrize("k", [512, 1024, 2048, 4096])
 def test_rows_of_zeros_and_overflow_take_the_usual_time(dev, k):
     """Padding rows, rows that start with zeros and denormal squares cost no more than ordinary rows
