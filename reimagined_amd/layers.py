@@ -52,9 +52,11 @@ class BitLinear:
     def gemm(self, q, s, m, y, st, magnitude=None, bias=None):
         """The ternary GEMM of m rows of codes into y: on the MFMA-layout words the MFMA GEMMs
         above 8 rows and at the skinny decode kernel's shapes, else the dispatching entry on
-        the reference words (GEMV / small-M MFMA kernels)."""
-        if self.packed_mfma is not None and (m > 8 or ops.skinny_shape(m, self.in_features,
-                                                                        self.out_features)):
+        the reference words (GEMV / small-M MFMA kernels; up to 128 rows also of a K past the
+        MFMA layout's sums)."""
+        few = 8 if self.in_features <= ops.MFMA_LAYOUT_MAX_K else 128
+        if self.packed_mfma is not None and (m > few or ops.skinny_shape(m, self.in_features,
+                                                                          self.out_features)):
             call("nsosx_ternary_gemm_mfma", _p(q), _p(s), _p(self.packed_mfma),
                  self.weight_scale, m, self.in_features, self.out_features, _p(magnitude),
                  _p(bias), _p(y), _DT[y.dtype], None, st)

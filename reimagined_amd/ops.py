@@ -136,6 +136,10 @@ def ternary_gemm(q: torch.Tensor, act_scale: torch.Tensor, packed: torch.Tensor,
     return y
 
 
+# Longest row of the MFMA layout's GEMMs, whose int32 sums are 64 times the ternary ones.
+MFMA_LAYOUT_MAX_K = 264208
+
+
 def skinny_shape(m: int, k: int, n: int) -> bool:
     """The shapes the skinny MFMA decode kernel takes (the library's skinny_ok): 2 <= m <=
     32, k in {1024, 2048, 4096}, ceil(m / 16) * k <= 4096, m * n * 4 < 2^31."""

@@ -522,3 +522,24 @@ def test_layer_bitlinear_decode_batches_bit_exact(dev, orc, m, k):
     y = lin.forward(torch.from_numpy(x).to(dev), out_dtype=torch.float32)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("m", [9, 16, 128, 129])
+def test_layer_rows_past_the_mfma_layouts_longest_row(dev, m):
+    """9 .. 128 rows of a K whose 64x sums leave int32 run on the reference words; more are refused."""
+    from reimagined_amd.layers import BitLinear
+    k, n = ops.MFMA_LAYOUT_MAX_K // 128 * 128 + 128, 20
+    rng = np.random.default_rng(m)
+    words = rng.integers(0, 2 ** 32, n * k // 16, dtype=np.uint64).astype(np.uint32)
+    words &= ~(words & (words >> 1) & np.uint32(0x55555555))
+    layer = BitLinear.from_packed(words, 1.0, n, k, device=dev)
+    q = torch.from_numpy(rng.integers(-127, 128, (m, k)).astype(np.int8)).to(dev)
+    y = torch.empty((m, n), device=dev)
+    run = lambda: layer.gemm(q, torch.ones(m, device=dev), m, y, None)
+    if m > 128:
+        with pytest.raises(Exception, match="too large"):
+            run()
+        return
+    run()
+    w = torch.from_numpy(ops.unpack_ternary(words, n * k).reshape(n, k)).to(dev)
+    assert torch.equal(y.double(), q.double() @ w.double().t().contiguous())  # (below 2^24: exact)
