@@ -525,28 +525,21 @@ class Mamba2Block:
         (nsosx_mamba2_step_out).  More rows: the quantization of u and the grouped x / z
         GEMV, the fp32 B / C / dt projection, the step, a norm launch and the out_proj."""
         m = u.shape[0]
-        # ops.mamba2_step's checks of the tensors that this block did not just make (with those of
-        # every projected view they took 15 us of host time per step)
-        cd = self.inner + 2 * self.gs
-        if self.K > 1:
-            ops._shape(ops._dev(dec["ring"], "ring", torch.float32), (m, self.K - 1, cd), "ring",
-                       "mamba2_step")
-        ops._shape(ops._dev(dec["state"], "state", torch.float32), (m, self.inner, self.N), "state",
-                   "mamba2_step")
-        for name, t, want in (("conv_w", self.conv_w_all, (cd, self.K)),
-                              ("conv_b", self.conv_b_all, (cd,)), ("a_log", self.a_log, (self.H,)),
-                              ("D", self.d_skip, (self.H,)), ("norm_w", self.norm_w, (self.inner,))):
-            if t.shape != want:
-                ops._shape(t, want, name, "mamba2_step")
+        op = self.out_proj
+        # ops.mamba2_step's checks but those of the projected views, which this block has just made
+        width = ops._mamba2_step_width(self.conv_w_all, self.conv_b_all,
+                                       dec["ring"] if self.K > 1 else None, self.a_log,
+                                       self.d_skip, self.norm_w, dec["state"], m, self.inner,
+                                       self.gs, self.H, self.N)
+        ops._mamba2_step_out_proj(op.packed, op.magnitude, op.bias, op.out_features, self.inner)
         xv, z, Bv, Cv, dt = self._project(u, contiguous_dt=False)
         q, s, _ = self.out_proj.workspace(m, u.device)
         y = torch.empty((m, self.inner), dtype=self.dtype, device=u.device)
-        op = self.out_proj
         out = torch.empty((m, op.out_features), dtype=self.dtype, device=u.device)
         # B, C and dt are column slices of one projection output, whose row stride they share
         call("nsosx_mamba2_step_out", _p(xv), _p(z), _p(Bv), _p(Cv), _p(dt), Bv.stride(0),
-             _p(self.conv_w_all), _p(self.conv_b_all), self.K,
-             _p(dec["ring"]) if self.K > 1 else None, _p(self.a_log), _p(self.d_skip),
+             _p(self.conv_w_all), _p(self.conv_b_all), width,
+             _p(dec["ring"]) if width > 1 else None, _p(self.a_log), _p(self.d_skip),
              _p(self.norm_w), self.eps, m, self.H, self.P, self.N, self.G, _DT[self.dtype],
              _p(dec["state"]), _p(y), _p(q), _p(s), op.bits, _p(op.packed), op.weight_scale,
              op.out_features, _p(op.magnitude), _p(op.bias), _p(out), _DT[self.dtype], _stream())

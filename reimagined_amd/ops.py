@@ -354,7 +354,7 @@ def grouped_gemv(views: LinearViewArray, q: torch.Tensor, act_scale: torch.Tenso
 # ---- Mamba ----------------------------------------------------------------------
 
 def _shape(t, want: tuple, name: str, fn: str) -> None:
-    if t is not None and tuple(t.shape) != tuple(want):
+    if t is not None and t.shape != tuple(want):
         raise ValueError(f"{fn}: {name} must have shape {tuple(want)}, got {tuple(t.shape)}")
 
 
@@ -510,6 +510,32 @@ def selective_scan_step(x, dt, a_log, B, C, D, z, state, H, P, N, G):
     return y
 
 
+def _mamba2_step_width(conv_w, conv_b, ring, a_log, D, norm_w, state, r, inner, gs, H, N) -> int:
+    """Checks mamba2_step's weights and states; returns the conv width."""
+    cd = inner + 2 * gs
+    _dev(conv_w, "conv_w", torch.float32)
+    width = conv_w.shape[1]
+    _shape(conv_w, (cd, width), "conv_w", "mamba2_step")
+    if conv_b is not None:
+        _shape(_dev(conv_b, "conv_b", torch.float32), (cd,), "conv_b", "mamba2_step")
+    if width > 1:
+        _shape(_dev(ring, "ring", torch.float32), (r, width - 1, cd), "ring", "mamba2_step")
+    _shape(_dev(a_log, "a_log", torch.float32), (H,), "a_log", "mamba2_step")
+    _shape(_dev(D, "D", torch.float32), (H,), "D", "mamba2_step")
+    if norm_w is not None:
+        _shape(_dev(norm_w, "norm_w", torch.float32), (inner,), "norm_w", "mamba2_step")
+    _shape(_dev(state, "state", torch.float32), (r, inner, N), "state", "mamba2_step")
+    return width
+
+
+def _mamba2_step_out_proj(packed, mag, bias, d, inner) -> None:
+    _dev(packed, "out_proj packed")
+    if packed.numel() != d * inner // 16:
+        raise ValueError("mamba2_step: out_proj weights must be [d, H*P/16] words and out [R, d]")
+    _opt(mag, "out_proj magnitude")
+    _opt(bias, "out_proj bias")
+
+
 def mamba2_step(x, z, B, C, dt, conv_w, conv_b, ring, a_log, D, norm_w, state, H, P, N, G,
                 eps: float = 1e-5, act_bits: int = 8, q=None, act_scale=None, y=None,
                 out_proj=None, out=None):
@@ -538,19 +564,7 @@ def mamba2_step(x, z, B, C, dt, conv_w, conv_b, ring, a_log, D, norm_w, state, H
                              "with unit column stride")
         if r > 1 and v.stride(0) != stride:
             raise ValueError("mamba2_step: B, C and dt must share one row stride")
-    cd = inner + 2 * gs
-    _dev(conv_w, "conv_w", torch.float32)
-    width = conv_w.shape[1]
-    _shape(conv_w, (cd, width), "conv_w", "mamba2_step")
-    if conv_b is not None:
-        _shape(_dev(conv_b, "conv_b", torch.float32), (cd,), "conv_b", "mamba2_step")
-    if width > 1:
-        _shape(_dev(ring, "ring", torch.float32), (r, width - 1, cd), "ring", "mamba2_step")
-    _shape(_dev(a_log, "a_log", torch.float32), (H,), "a_log", "mamba2_step")
-    _shape(_dev(D, "D", torch.float32), (H,), "D", "mamba2_step")
-    if norm_w is not None:
-        _shape(_dev(norm_w, "norm_w", torch.float32), (inner,), "norm_w", "mamba2_step")
-    _shape(_dev(state, "state", torch.float32), (r, inner, N), "state", "mamba2_step")
+    width = _mamba2_step_width(conv_w, conv_b, ring, a_log, D, norm_w, state, r, inner, gs, H, N)
     if q is None:
         q = torch.empty((r, inner), dtype=torch.int8, device=x.device)
     if act_scale is None:
@@ -567,12 +581,10 @@ def mamba2_step(x, z, B, C, dt, conv_w, conv_b, ring, a_log, D, norm_w, state, H
         call("nsosx_mamba2_step", *args, _stream())
         return q, act_scale, y
     packed, ws, mag, bias = out_proj
-    _dev(packed, "out_proj packed")
     d = out.shape[1]
-    if packed.numel() != d * inner // 16 or tuple(out.shape) != (r, d) or not out.is_contiguous():
+    if tuple(out.shape) != (r, d) or not out.is_contiguous():
         raise ValueError("mamba2_step: out_proj weights must be [d, H*P/16] words and out [R, d]")
-    _opt(mag, "out_proj magnitude")
-    _opt(bias, "out_proj bias")
+    _mamba2_step_out_proj(packed, mag, bias, d, inner)
     call("nsosx_mamba2_step_out", *args, _p(packed), ws, d, _p(mag), _p(bias), _p(out), _dt(out),
          _stream())
     return q, act_scale, y

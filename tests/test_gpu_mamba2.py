@@ -331,3 +331,27 @@ def test_mamba2_step_out_equals_step_then_gemm(dev, R, H, P, N, G, W, dtype, d):
         res.append([t.float().cpu().numpy() for t in (out, q, s, state, ring, y)])
     for want, got in zip(*res):
         np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_mamba2_step_refuses_replaced_weights(dev, rows):
+    """A weight or state replaced by one of another type, stride, shape or device is refused, and the
+    states stay as they were."""
+    blk = Mamba2Block(_params(np.random.default_rng(1)), dev)
+    u = torch.randn((rows, 64), device=dev)
+    names = ("conv_w_all", "conv_b_all", "a_log", "d_skip", "norm_w")
+    for name in names + ("state", "ring", "packed"):
+        dec = blk.new_decode_state(rows, dev)
+        at, key = ((dec, name) if name in dec else
+                   (blk.out_proj.__dict__ if name == "packed" else blk.__dict__, name))
+        good = at[key]
+        bad = [good[:-1].contiguous(), good.cpu()]
+        if name != "packed":
+            bad += [good.to(torch.bfloat16), torch.stack([good, good], -1)[..., 0]]
+        for t in bad:
+            at[key] = t
+            with pytest.raises(ValueError):
+                blk.step(u, dec)
+        at[key] = good
+    want = blk.step(u, blk.new_decode_state(rows, dev))
+    assert torch.isfinite(want).all()
