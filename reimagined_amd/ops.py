@@ -29,10 +29,15 @@ def _p(t):
     return None if t is None else t.data_ptr()
 
 
+# torch's current stream handle without a torch.cuda.Stream built around it (1.5 us of host time
+# per launch); not part of its public interface
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
-    # the current stream's handle without building a torch.cuda.Stream around it (1.5 us of
-    # host time per launch)
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> torch.Tensor:

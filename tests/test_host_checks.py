@@ -183,3 +183,19 @@ def test_grouped_mfma_ws_argument_checks():
     rc = L.nsosx_grouped_ternary_gemm_mfma_ws(_FAKE, 8, _FAKE, _FAKE, 1, _FAKE, _FAKE, 1000,
                                               4096, 100, 1, _FAKE, 1, _FAKE, 1 << 26, None)
     assert rc == 1 and b"K % 128" in L.nsosx_last_error()
+
+
+def test_stream_handle_without_torchs_short_way(monkeypatch):
+    """Where torch lacks the raw handle's function the public stream gives it."""
+    from types import SimpleNamespace
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=7))
+    assert ops._stream() == 7
+
+
+@pytest.mark.gpu
+def test_stream_handle_is_the_current_streams(dev):
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert ops._stream() == side.cuda_stream
