@@ -131,10 +131,11 @@ int nsosx_quantize_act_i8(const void* x, int x_dtype, int M, int K, int bits, in
  * Replaces launch_bitnet_gemm / launch_bitnet_gemv_scaled /
  * launch_bitnet_apply_act_scales_kernel (include/cuda/kernels.cuh:106-110).
  * M = 1 runs the packed-weight streaming GEMV; K % 128 == 0 and N <= 16384 the
- * int8 MFMA GEMMs (small tiles where 256 x 128 ones would leave CUs idle);
- * otherwise 2 <= M <= 32 with K in {1024, 2048, 4096} (ceil(M/16) * K <= 4096)
- * the skinny MFMA kernel (one decoded word feeds 16 tokens); other M <= 8 the
- * GEMV; larger M the int8 MFMA GEMMs.
+ * int8 MFMA GEMMs (small tiles where 256 x 128 ones would leave CUs idle; two
+ * to four rows of a long K stay on the GEMV); otherwise 2 <= M <= 32 with K in
+ * {1024, 2048, 4096} (ceil(M/16) * K <= 4096) the skinny MFMA kernel (one
+ * decoded word feeds 16 tokens); other M <= 8 the GEMV; larger M the int8 MFMA
+ * GEMMs.
  *   y: [M, N] f32 or bf16 (y_dtype), may be NULL when acc_out is given.
  *   acc_out: int32 [M, N] or NULL (exposes the accumulators).
  *   magnitude, bias: f32 [N] or NULL. */

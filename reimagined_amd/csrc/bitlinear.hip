@@ -60,12 +60,22 @@ static int check_gemm_args(const int8_t* q, const float* as, const uint32_t* pac
     return NSOSX_OK;
 }
 
+// Two to four rows of a long K, where the small tiles' four waves share few columns and the GEMV's
+// lanes the whole row.  2 rows, GEMV / small tiles, us, weights from HBM: K 2560, N 4096 4.5 / 4.9;
+// 5120 x 4096 6.2 / 7.6; 8192 x 16384 11.9 / 14.6; but 2560 x 16384 7.1 / 6.9, 1536 x 4096
+// 4.3 / 4.1.  3 rows: 8192 x 1024 7.0 / 9.0; 8192 x 4096 9.5 / 9.4, 5120 x 1024 6.7 / 6.6.
+static bool gemv_rows(int M, int K, int N) {
+    if (M == 2) return K > 2048 && (N <= 8192 || K >= 8192);
+    return M <= 4 && K >= 8192 && N <= 2048;
+}
+
 // M = 1: the VALU GEMV; a matrix the caches hold (K % 128 == 0, N <= kSmallMaxN): the
-// MFMA GEMMs, whose small tiles take it; 2 <= M <= 32 where the skinny MFMA path takes
-// the shape; other M <= 8: the GEMV; else the MFMA GEMM.
+// MFMA GEMMs, whose small tiles take it (but gemv_rows); 2 <= M <= 32 where the skinny MFMA path
+// takes the shape; other M <= 8: the GEMV; else the MFMA GEMM.
 static int ternary_gemm_auto_path(int M, int K, int N) {
-    if (M > 1 && K % kG3BK == 0 && N <= kSmallMaxN) return 1;
-    if (skinny_ok(M, K, N)) return 2;
+    const bool skinny = skinny_ok(M, K, N);
+    if (M > 1 && K % kG3BK == 0 && N <= kSmallMaxN && (skinny || !gemv_rows(M, K, N))) return 1;
+    if (skinny) return 2;
     return M <= 8 ? 0 : 1;
 }
 

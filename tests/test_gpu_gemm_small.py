@@ -85,3 +85,19 @@ def test_grouped_small_tiles_bit_exact(dev, rows, k, n, gather):
                 v = v * v
             want[seg] = v
         np.testing.assert_array_equal(y.cpu().numpy(), want)
+
+
+# Either side of the rule that keeps few rows of a long K on the GEMV
+@pytest.mark.parametrize("m,k,n", [(2, 2048, 68), (2, 2176, 68), (2, 2176, 8192), (2, 2176, 8196),
+                                   (2, 8192, 8196), (3, 8064, 36), (4, 8192, 2048), (4, 8192, 2052),
+                                   (5, 8192, 68)])
+def test_few_rows_of_long_k_bit_exact(dev, m, k, n):
+    rng = np.random.default_rng(m + k + n)
+    codes, words = _matrix(rng, n, k)
+    q = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    s = rng.uniform(0.01, 0.1, m).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    y, acc = ops.ternary_gemm(t(q), t(s), t(words.view(np.int32)), 0.37, n, want_acc=True)
+    want = np.rint(q.astype(np.float64) @ codes.T.astype(np.float64)).astype(np.int32)
+    np.testing.assert_array_equal(acc.cpu().numpy(), want)
+    np.testing.assert_array_equal(y.cpu().numpy(), _affine(want, s, 0.37, None, None))
