@@ -24,7 +24,7 @@ def _affine(acc, s, ws, mag, bias):
 
 
 # K of 1, 2, 3, 4, 5 and 9 blocks of 128 (waves with no block, uneven quarters); row counts and
-# widths on either side of 32 / 64; 2048 x 3 000-odd rows past the point where large tiles win
+# widths on either side of 32 / 64; 3001 rows, the most that the 64 x 64 tiles take here
 @pytest.mark.parametrize("m,k,n", [(2, 128, 32), (9, 256, 33), (31, 384, 7), (32, 512, 64),
                                    (33, 640, 100), (64, 1152, 129), (65, 128, 768), (100, 2048, 8192),
                                    (300, 768, 768), (257, 1024, 4104), (700, 2048, 1000),
@@ -85,6 +85,22 @@ def test_grouped_small_tiles_bit_exact(dev, rows, k, n, gather):
                 v = v * v
             want[seg] = v
         np.testing.assert_array_equal(y.cpu().numpy(), want)
+
+
+# The last row counts of the small tiles and the first of the 256 x 128 ones at one width (by the
+# rule 143 against 174 tenths of a us, then 192 against 174)
+@pytest.mark.parametrize("m", [200, 300])
+@pytest.mark.parametrize("mfma", [True, False])
+def test_either_side_of_the_rule_bit_exact(dev, m, mfma):
+    test_small_tiles_bit_exact(dev, m, 2048, 8192, mfma, torch.float32)
+
+
+# 64 x 64 tiles per expert (rows around a multiple of 64, an expert without rows, a width that is
+# not one), which the cases above never pick
+@pytest.mark.parametrize("k,n", [(1024, 2000), (2048, 1000)])
+@pytest.mark.parametrize("gather", [True, False])
+def test_grouped_64_by_64_tiles_bit_exact(dev, k, n, gather):
+    test_grouped_small_tiles_bit_exact(dev, [200, 130, 64, 0, 65, 241], k, n, gather)
 
 
 # Either side of the rule that keeps few rows of a long K on the GEMV
