@@ -86,9 +86,11 @@ void launch_grouped_skinny(dim3 grid, const nsosx_linear_view* views, const int8
                            void* y, int64_t y_stride, int y_dtype, hipStream_t st);
 // gemm_small.hip: outputs too small for the 256 x 128 tiles (K % 128 == 0), on either layout;
 // false where those are the faster ones (nothing launched).  kSmallMaxN: up to here the
-// small tiles also beat the skinny kernel and the GEMV at 2 .. 32 rows (measured at K 1024 /
-// 2048 / 4096: 3.2 / 3.8 / 5.0 us against 3.9 / 6.0 / 9.8); on larger matrices, which stream
-// their weights from HBM, the skinny kernel's four times smaller load traffic wins.
+// small tiles also beat the skinny kernel and, but for few rows of a long K, the GEMV at 2 .. 32
+// rows (4 rows of K 1024 / 2048 / 4096, N 4096 / 8192 / 4096: 3.3 / 3.8 / 4.8 us against 3.9 / 6.1 /
+// 10.4; with the weights from HBM 3.9 / 4.7 / 5.8 against 4.0 / 6.8 / 10.7; N 16384, K 4096 from
+// HBM 8.4 against 12.2).  The stacked matrices of a decode sweep, far wider, stay with the skinny
+// kernel and its four times smaller load traffic.
 constexpr int kSmallMaxN = 16384;
 bool launch_gemm_small(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,
                        int y_dtype, int32_t* acc, bool mfma_layout, hipStream_t st);

@@ -216,7 +216,9 @@ __global__ __launch_bounds__(256) void grouped_gemm_small_kernel(
 // tile takes 0.8 us per block and its rounds are 256 or more tiles.  Measured, us (small /
 // 256 x 128 tiles): K 2048, N 8192: 64 rows 5.8 / 17 (and 41 on the old few-row kernel),
 // 200 rows 14.5 / 17.6, 300 rows 19.6 / 17.7; K 4096, N 1024: 64 rows 7.3 / 30, 1500 rows
-// 20.5 / 30.5, 3000 rows 33 / 31.
+// 20.5 / 30.5, 3000 rows 33 / 31.  Weights from HBM add about as much to either side and leave
+// the rule where it is: K 2048, N 8192: 64 rows 7.0 / 19.2, 200 rows 15.7 / 19.1; 64 routed rows over
+// 8 experts, 1024 -> 4096 -> 1024: 7.4 / 9.8 up, 9.0 / 29.3 down; 256 rows 12.9 / 12.8, 16 / 38.5.
 struct SmallChoice {
     int nt, mt;  // 0: the 256 x 128 kernel
 };

@@ -10,9 +10,9 @@
 // sixteenth of the matrix-core time per pass.  Before: two fp32-MFMA GEMMs at the
 // card's fp32 rate (400 + 407 us at M = 4096, K = 1024, N = 4096), a full ternary
 // GEMM for dmag (27 us) and a column reduction over two [M, N] arrays (145 us).  Now one
-// launch of about 220 us for both contractions and the column sums (MFMA issue alone: 94 us at
-// the ~2.1 GHz it runs at; dW's strided gradient reads and its epilogue make its tiles the
-// longer ones), a forward and backward step 1062 -> 273 us.
+// launch of 230 us (200 where it runs alone) for both contractions and the column sums (MFMA issue
+// alone: 94 us at the ~2.1 GHz it runs at; dW's strided gradient reads and its epilogue make its
+// tiles the longer ones), a forward and backward step 1059 -> 268 us.
 #include "row_sum.hpp"
 
 #include <algorithm>
@@ -616,9 +616,7 @@ __global__ __launch_bounds__(512) void rms_backward_row_kernel(const void* __res
 
 static int64_t round256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
-// Row pitch of the transposed operands: whole 256-byte units, an odd number of them, so
-// that a tile's 256 rows (64 bytes of each per stage) spread over the L2 channels; a
-// power-of-two pitch puts them all on one.
+// Row pitch of the transposed operands: whole stages of the reduction.
 static int ste_pitch(int n) { return (n + kTK - 1) / kTK * kTK; }
 
 struct SteWorkspace {
