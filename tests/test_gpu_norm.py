@@ -149,3 +149,17 @@ def test_rmsnorm_gated_quant_equals_two_passes(dev, orc, rows, dim, dtype, keep)
     wq, ws = orc.quantize_act(normed.float().cpu().numpy(), 8)
     np.testing.assert_array_equal(q.cpu().numpy(), wq)
     np.testing.assert_array_equal(s.cpu().numpy(), ws)
+
+
+@pytest.mark.parametrize("dim", [1, 63, 64, 65, 128, 129, 256, 257, 768, 769])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_add_rmsnorm_short_rows(dev, orc, dim, dtype):
+    test_add_rmsnorm_row_lengths(dev, orc, dim, dtype)
+
+
+@pytest.mark.parametrize("dim", [64, 1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_residual_add_without_norm(dev, dim, dtype):
+    x, d = (torch.randn((5, dim), device=dev).to(dtype) for _ in range(2))
+    res, none = ops.add_rmsnorm(x, d, want_norm=False)
+    assert none is None and torch.equal(res, (x.float() + d.float()).to(dtype))
