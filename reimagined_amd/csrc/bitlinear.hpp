@@ -95,10 +95,10 @@ constexpr int kSmallMaxN = 16384;
 bool launch_gemm_small(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,
                        int y_dtype, int32_t* acc, bool mfma_layout, hipStream_t st);
 // the experts' row segments, MFMA layout (perm null: rows already in slot order);
-// large_extra: what the tiled launch would cost besides its tiles, in 0.1 us
+// split: whether the tiled launch would be the one with a split tail
 bool launch_grouped_gemm_small(const nsosx_linear_view* views, int experts, const int32_t* offsets,
                                const int32_t* perm, const int8_t* q, const float* as, int K, int N,
-                               int total_rows, int sqrelu, void* y, int y_dtype, double large_extra,
+                               int total_rows, int sqrelu, void* y, int y_dtype, bool split,
                                hipStream_t st);
 // gemm.hip: the MFMA GEMMs on the reference words and on the MFMA layout
 void launch_gemm(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,

@@ -234,10 +234,9 @@ extern "C" int nsosx_grouped_ternary_gemm_mfma_ws(const nsosx_linear_view* views
                                                act_scale, K, N, total_rows, squared_relu, y,
                                                y_dtype, stream);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // few rows per expert: small tiles (the split launch costs its fixup and about 10 us over
-    // its tiles: 40 us against 23 at 1024 rows of 4096 over 8 experts)
+    // few rows per expert: small tiles (24 us against 41 at 1000 rows of 4096 over 8 experts)
     if (launch_grouped_gemm_small(views_dev, experts, offsets, gather ? perm : nullptr, q, act_scale,
-                                  K, N, total_rows, squared_relu, y, y_dtype, 100.0, st))
+                                  K, N, total_rows, squared_relu, y, y_dtype, true, st))
         return check_launch("grouped_ternary_gemm_mfma_ws");
     int32_t* raw = static_cast<int32_t*>(workspace);
 #define NSOSX_GGS(YDT, G, S)                                                                     \
@@ -283,7 +282,7 @@ extern "C" int nsosx_grouped_ternary_gemm_mfma(const nsosx_linear_view* views_de
         return fail(NSOSX_ERR_INVALID, "grouped_ternary_gemm_mfma: too many tiles");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (launch_grouped_gemm_small(views_dev, experts, offsets, gather ? perm : nullptr, q, act_scale,
-                                  K, N, total_rows, squared_relu, y, y_dtype, 0.0, st))
+                                  K, N, total_rows, squared_relu, y, y_dtype, false, st))
         return check_launch("grouped_ternary_gemm_mfma");
 #define NSOSX_GGM(YDT, G, S)                                                                     \
     hipLaunchKernelGGL((grouped_gemm3_mfma_kernel<YDT, G, S>), dim3(ntn * ntm), dim3(kGemm3Threads),   \

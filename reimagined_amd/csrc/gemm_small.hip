@@ -212,8 +212,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_small_kernel(
 // Which kernel takes a shape: the estimated time of each in 0.1 us, from a sweep of K 768 ..
 // 4096, N 768 .. 16384 and 9 .. 3000 rows (weights in the caches).  A small-tile launch runs
 // in rounds of 256 workgroups (one per CU; more per CU only overlap, their loads share the
-// vector cache), each a term per 128-deep block of K and a fixed one; the 256 x 128 kernel's
-// tile takes 0.8 us per block and its rounds are 256 or more tiles.  Measured, us (small /
+// vector cache), each a term per 128-deep block of K and a fixed one; 256 of the 256 x 128 kernel's
+// tiles take 0.19 us per block and 0.28 more per 32 rows that they hold.  Measured, us (small /
 // 256 x 128 tiles): K 2048, N 8192: 64 rows 5.8 / 17 (and 41 on the old few-row kernel),
 // 200 rows 14.5 / 17.6, 300 rows 19.6 / 17.7; K 4096, N 1024: 64 rows 7.3 / 30, 1500 rows
 // 20.5 / 30.5, 3000 rows 33 / 31.  Weights from HBM add about as much to either side and leave
@@ -224,14 +224,15 @@ struct SmallChoice {
 };
 
 static SmallChoice small_choice(int K, int N, double rows32, double rows64, double rows128,
-                                double large_extra) {
+                                double large_extra, double small_extra) {
     const double kb = K / kG3BK;
     const double n32 = (N + 31) / 32, n64 = (N + 63) / 64, n256 = (N + kG3BN - 1) / kG3BN;
     auto rounds = [](double tiles) { return std::ceil(tiles / 256.0); };
-    const double c11 = 22 + rounds(n32 * rows32) * (5.5 + 1.46 * kb);
-    const double c21 = 22 + rounds(n64 * rows32) * (6.0 + 1.75 * kb);
-    const double c22 = 22 + rounds(n64 * rows64) * (18.0 + 2.65 * kb);
-    const double large = std::max(46 + 8.0 * kb, n256 * rows128 * kb / 20) + large_extra;
+    const double c11 = 22 + small_extra + rounds(n32 * rows32) * (5.5 + 1.46 * kb);
+    const double c21 = 22 + small_extra + rounds(n64 * rows32) * (6.0 + 1.75 * kb);
+    const double c22 = 22 + small_extra + rounds(n64 * rows64) * (18.0 + 2.65 * kb);
+    const double large =
+        46 + std::max(8.0 * kb, n256 * kb * (1.9 * rows128 + 2.8 * rows32) / 256) + large_extra;
     const double best = std::min(std::min(c11, c21), c22);
     if (large <= best) return {0, 0};
     if (c11 == best) return {1, 1};
@@ -241,7 +242,7 @@ static SmallChoice small_choice(int K, int N, double rows32, double rows64, doub
 template <bool SWZ>
 static bool launch_small_t(const GemmProblem& pb, const int8_t* q, const float* as, int M, void* y,
                            int y_dtype, int32_t* acc, hipStream_t st) {
-    const SmallChoice c = small_choice(pb.K, pb.N, (M + 31) / 32, (M + 63) / 64, (M + 127) / 128, 0.0);
+    const SmallChoice c = small_choice(pb.K, pb.N, (M + 31) / 32, (M + 63) / 64, (M + 127) / 128, 0, 0);
     if (c.nt == 0) return false;
     const int ybf = y_dtype == NSOSX_BF16;
 #define NSOSX_SMALL(NT, MT)                                                                     \
@@ -263,18 +264,26 @@ bool launch_gemm_small(const GemmProblem& pb, const int8_t* q, const float* as, 
 }
 
 // The experts' row counts are on the device: each expert's last tile is taken as three
-// quarters of a tile more than its share.
+// quarters of a tile more than its share.  The large kernel's workgroups find their segment in 0.1 us
+// per expert, and its split launch takes about 4 us and 0.45 per expert more (ws against not, 4096 x
+// 512, 1000 rows: 2 experts 36.9 / 32.7, 16 40.1 / 29.1, 64 62.8 / 30.8).  The small tiles read the
+// codes on every XCD, which past 8 MB (two L2s) takes its time: 5000 rows of 4096, 512 outputs,
+// 8 experts 48.2 us small, 42.8 large.
 bool launch_grouped_gemm_small(const nsosx_linear_view* views, int experts, const int32_t* offsets,
                                const int32_t* perm, const int8_t* q, const float* as, int K, int N,
-                               int total_rows, int sqrelu, void* y, int y_dtype, double large_extra,
+                               int total_rows, int sqrelu, void* y, int y_dtype, bool split,
                                hipStream_t st) {
     auto tiles = [&](int rows) {
         return std::min<double>(total_rows, std::ceil((double)total_rows / rows + 0.75 * experts));
     };
-    const SmallChoice c = small_choice(K, N, tiles(32), tiles(64), tiles(128), large_extra);
+    const double codes = std::max(0.0, (double)total_rows * K - 8e6) * 8e-6;  // 10 TB/s, eight XCDs
+    const double large_extra = experts + (split ? 40 + 4.5 * experts : 0);
+    const SmallChoice c = small_choice(K, N, tiles(32), tiles(64), tiles(128), large_extra, codes);
     if (c.nt == 0) return false;
     const int ntn = (N + 32 * c.nt - 1) / (32 * c.nt);
-    const int ntm = (total_rows + 32 * c.mt - 1) / (32 * c.mt) + experts;  // >= the real row tiles
+    // >= the real row tiles, each of which holds a row (a workgroup past them walks every expert: 2
+    // rows, 64 experts, 1024 -> 4096 63 us without the bound, 7.1 with it)
+    const int ntm = std::min(total_rows, (total_rows + 32 * c.mt - 1) / (32 * c.mt) + experts);
     if ((int64_t)ntn * ntm > 0x7fffffff) return false;
     const int ybf = y_dtype == NSOSX_BF16;
 #define NSOSX_SMALL(NT, MT)                                                                       \

@@ -117,3 +117,12 @@ def test_few_rows_of_long_k_bit_exact(dev, m, k, n):
     want = np.rint(q.astype(np.float64) @ codes.T.astype(np.float64)).astype(np.int32)
     np.testing.assert_array_equal(acc.cpu().numpy(), want)
     np.testing.assert_array_equal(y.cpu().numpy(), _affine(want, s, 0.37, None, None))
+
+
+# More experts than a wave has lanes, most of them without rows: the first, the last, at a multiple
+# of 64 and past it
+@pytest.mark.parametrize("rows", [{0: 1, 1: 33}, {63: 40, 64: 2, 69: 31}, {127: 5, 128: 70, 129: 1},
+                                  {e: e % 3 for e in range(130)}])
+@pytest.mark.parametrize("gather", [True, False])
+def test_grouped_many_experts_bit_exact(dev, rows, gather):
+    test_grouped_small_tiles_bit_exact(dev, [rows.get(e, 0) for e in range(130)], 128, 96, gather)
