@@ -520,16 +520,15 @@ def _mamba2_step_width(conv_w, conv_b, ring, a_log, D, norm_w, state, r, inner, 
     cd = inner + 2 * gs
     _dev(conv_w, "conv_w", torch.float32)
     width = conv_w.shape[1]
-    _shape(conv_w, (cd, width), "conv_w", "mamba2_step")
-    if conv_b is not None:
-        _shape(_dev(conv_b, "conv_b", torch.float32), (cd,), "conv_b", "mamba2_step")
-    if width > 1:
-        _shape(_dev(ring, "ring", torch.float32), (r, width - 1, cd), "ring", "mamba2_step")
-    _shape(_dev(a_log, "a_log", torch.float32), (H,), "a_log", "mamba2_step")
-    _shape(_dev(D, "D", torch.float32), (H,), "D", "mamba2_step")
-    if norm_w is not None:
-        _shape(_dev(norm_w, "norm_w", torch.float32), (inner,), "norm_w", "mamba2_step")
-    _shape(_dev(state, "state", torch.float32), (r, inner, N), "state", "mamba2_step")
+    for name, t, want in (("conv_w", conv_w, (cd, width)), ("conv_b", conv_b, (cd,)),
+                          ("ring", ring if width > 1 else None, (r, width - 1, cd)),
+                          ("a_log", a_log, (H,)), ("D", D, (H,)), ("norm_w", norm_w, (inner,)),
+                          ("state", state, (r, inner, N))):
+        if t is None and (name in ("conv_b", "norm_w") or (name == "ring" and width <= 1)):
+            continue
+        # (one line where all is well: a decode step runs this on every call)
+        if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.shape == want):
+            _shape(_dev(t, name, torch.float32), want, name, "mamba2_step")
     return width
 
 
