@@ -240,7 +240,7 @@ int nsosx_linear_f32(const void* x, int x_dtype, int M, int K, const float* w, i
  * nsosx_bitlinear_ste_backward_workspace(M, K, N, rms_input) bytes, 256-byte
  * aligned.  Sums run in fp32 in an order of their own (tolerance parity).
  * Outputs may lie over grad and magnitude; dW over w_latent; dx over q, act_scale or
- * w_latent, or with rms_input over x.  They must not overlap other inputs, each
+ * w_latent, or with rms_input over an f32 x.  They must not overlap other inputs, each
  * other or the workspace. */
 int64_t nsosx_bitlinear_ste_backward_workspace(int M, int K, int N, int rms_input);
 int nsosx_bitlinear_ste_backward(const void* x, int x_dtype, const int8_t* q,
